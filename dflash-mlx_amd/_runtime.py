@@ -94,6 +94,14 @@ class _WorkspaceCache:
         self.get(device, nbytes, kind)
 
 
+    def held(self, device: torch.device, kind: str = "qmm") -> Optional[torch.Tensor]:
+        """This stream's buffer as it is, or None."""
+        key = (device.index if device.index is not None else torch.cuda.current_device(),
+               stream_ptr(device), kind)
+        with self._lock:
+            return self._bufs.get(key)
+
+
 WORKSPACES = _WorkspaceCache()
 
 
@@ -103,6 +111,26 @@ def workspace(device: torch.device, nbytes: int, kind: str = "qmm") -> tuple[int
     base = buf.data_ptr()
     aligned = (base + 255) // 256 * 256
     return aligned, buf.numel() - (aligned - base)
+
+
+def optional_workspace(device: torch.device, nbytes: int, kind: str = "qmm") -> tuple[int, int]:
+    """:func:`workspace` for a call that also runs with less: while a graph is
+    being captured, when nothing may grow, what the stream holds already (or
+    (0, 0))."""
+    if torch.cuda.is_current_stream_capturing():
+        buf = WORKSPACES.held(device, kind)
+        if buf is None:
+            return 0, 0
+        base = buf.data_ptr()
+        aligned = (base + 255) // 256 * 256
+        return aligned, buf.numel() - (aligned - base)
+    return workspace(device, nbytes, kind)
+
+
+def many_rows(M: int) -> bool:
+    """Row counts above the streaming kernels' (``qmm_gemm_kernel``): the
+    launch reads a pair table at every group size, bit width and K."""
+    return int(M) > 32
 
 
 def pair_shape(M: int, K: int, N: int, group_size: int, bits: int) -> bool:

@@ -1,0 +1,8 @@
+// qmm_gemm_kernel for bf16 activations and 4-bit weights.
+#include "dfmi_gemm.h"
+
+namespace dfmi {
+void gemm_launch_bf16_4(int cfg, int gs, const GemmArgs& a, hipStream_t st) {
+  gemm_launch_bits<BF16, 4>(cfg, gs, a, st);
+}
+}  // namespace dfmi

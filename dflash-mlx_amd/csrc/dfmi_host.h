@@ -35,6 +35,18 @@ inline bool stream_eligible(int64_t M, int64_t K, int64_t N, int gs, int bits = 
          N * (K / 8 * bits) < (1ll << 31);
 }
 
+// Many activation rows (dfmi_gemm.hip).  The workspace holds the streaming
+// kernels' counters (untouched), the pair table of a call without one, and
+// the partial tiles of a K split; with less of it (or none) the call runs
+// unsplit, or, without a table either, is not taken.
+constexpr int kGemmNotTaken = 1;
+bool gemm_shape(int64_t M, int64_t K, int64_t N, int gs);
+size_t gemm_workspace_bytes(int64_t M, int64_t K, int64_t N, int gs);
+int gemm_launch(const void* x, int x_dtype, const uint32_t* w, const void* scales,
+                const void* biases, const uint32_t* pairs, int64_t pair_stride, void* y,
+                int64_t M, int64_t K, int64_t N, int gs, int bits, void* workspace,
+                size_t workspace_bytes, hipStream_t st);
+
 }  // namespace dfmi
 
 // 8-bit affine qmm launch (dfmi_qmm8.hip), called by dfmi_qmm_affine_ex after

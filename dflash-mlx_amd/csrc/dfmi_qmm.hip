@@ -968,11 +968,19 @@ static int64_t multi_stream_cols(int64_t M, int64_t K, const int64_t* Ns, int ns
   return blocks * kStreamRows;
 }
 
+// The matrix-core kernel for many rows is the automatic choice above the
+// streaming kernels' 32 rows (a forced general plan keeps the general kernel).
+static bool use_gemm(int64_t M, int64_t K, int64_t N, int gs, const dfmi_qmm_tuning* tune) {
+  return gemm_shape(M, K, N, gs) &&
+         (!tune || (tune->path == 0 && !tune->tiles_per_wave && !tune->waves_per_block));
+}
+
 extern "C" size_t dfmi_qmm_workspace_bytes_ex(int64_t M, int64_t K, int64_t N, int group_size,
                                               int bits, const dfmi_qmm_tuning* tuning) {
   if (validate_qmm(DFMI_BF16, M, K, N, group_size, bits) != DFMI_OK || M == 0 || N == 0 ||
       !valid_path(tuning))
     return 0;
+  if (use_gemm(M, K, N, group_size, tuning)) return gemm_workspace_bytes(M, K, N, group_size);
   if (!use_stream(M, K, N, group_size, bits, tuning)) return 0;
   StreamPlan p;
   if (plan_stream(M, K, N, group_size, bits, tuning, p) != DFMI_OK) return 0;
@@ -1018,6 +1026,7 @@ extern "C" const char* dfmi_qmm_kernel_name(int64_t M, int64_t K, int64_t N, int
                                              int bits, const dfmi_qmm_tuning* tuning) {
   if (validate_qmm(DFMI_BF16, M, K, N, group_size, bits) != DFMI_OK || !valid_path(tuning))
     return nullptr;
+  if (use_gemm(M, K, N, group_size, tuning)) return "qmm_gemm_kernel";
   if (bits == 8) return use_stream(M, K, N, group_size, bits, tuning) ? "qmm8_stream_kernel"
                                                                       : "qmm8_kernel";
   return use_stream(M, K, N, group_size, bits, tuning) ? "qmm_stream_kernel" : "qmm_dense_kernel";
@@ -1028,12 +1037,11 @@ extern "C" size_t dfmi_qmm_workspace_bytes(int64_t M, int64_t K, int64_t N, int 
   return dfmi_qmm_workspace_bytes_ex(M, K, N, group_size, bits, nullptr);
 }
 
-extern "C" int dfmi_qmm_affine_pairs(const void* x, int x_dtype, const uint32_t* w_q,
-                                     const void* scales, const void* biases,
-                                     const uint32_t* sb_pairs, void* y, int64_t M, int64_t K,
-                                     int64_t N, int group_size, int bits, void* workspace,
-                                     size_t workspace_bytes, const dfmi_qmm_tuning* tuning,
-                                     void* stream) {
+// dfmi_qmm_affine_pairs; sb_stride: the pair table's row length (0: N)
+static int qmm_affine(const void* x, int x_dtype, const uint32_t* w_q, const void* scales,
+                      const void* biases, const uint32_t* sb_pairs, int64_t sb_stride, void* y,
+                      int64_t M, int64_t K, int64_t N, int group_size, int bits, void* workspace,
+                      size_t workspace_bytes, const dfmi_qmm_tuning* tuning, void* stream) {
   int rc = validate_qmm(x_dtype, M, K, N, group_size, bits);
   if (rc != DFMI_OK) return rc;
   if (!valid_path(tuning)) {
@@ -1059,6 +1067,11 @@ extern "C" int dfmi_qmm_affine_pairs(const void* x, int x_dtype, const uint32_t*
     return DFMI_EINVAL;
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (use_gemm(M, K, N, group_size, tuning)) {
+    rc = gemm_launch(x, x_dtype, w_q, scales, biases, sb_pairs, sb_stride, y, M, K, N, group_size,
+                     bits, workspace, workspace_bytes, st);
+    if (rc != kGemmNotTaken) return rc;
+  }
   // 8-bit: the streaming kernel where it applies, else the register-load kernel
   if (bits == 8 && !use_stream(M, K, N, group_size, bits, tuning))
     return dfmi_qmm8_launch(x, x_dtype, w_q, scales, biases, y, M, K, N, group_size, stream);
@@ -1068,6 +1081,7 @@ extern "C" int dfmi_qmm_affine_pairs(const void* x, int x_dtype, const uint32_t*
                          static_cast<const uint16_t*>(biases), static_cast<uint16_t*>(y), (int)N, 0,
                          sb_pairs};
     m.nseg = 1;
+    m.tn = (uint32_t)sb_stride;
     return launch_streaming(x, x_dtype, m, M, K, N, group_size, bits, tuning, workspace,
                             workspace_bytes, st);
   }
@@ -1087,6 +1101,32 @@ extern "C" int dfmi_qmm_affine_pairs(const void* x, int x_dtype, const uint32_t*
   if (x_dtype == DFMI_BF16) launch_tag<BF16>(group_size, p, st, a);
   else launch_tag<F16>(group_size, p, st, a);
   return check_launch("dfmi_qmm_affine");
+}
+
+extern "C" int dfmi_qmm_affine_pairs(const void* x, int x_dtype, const uint32_t* w_q,
+                                     const void* scales, const void* biases,
+                                     const uint32_t* sb_pairs, void* y, int64_t M, int64_t K,
+                                     int64_t N, int group_size, int bits, void* workspace,
+                                     size_t workspace_bytes, const dfmi_qmm_tuning* tuning,
+                                     void* stream) {
+  return qmm_affine(x, x_dtype, w_q, scales, biases, sb_pairs, 0, y, M, K, N, group_size, bits,
+                    workspace, workspace_bytes, tuning, stream);
+}
+
+extern "C" int dfmi_qmm_affine_pairs_strided(const void* x, int x_dtype, const uint32_t* w_q,
+                                             const void* scales, const void* biases,
+                                             const uint32_t* sb_pairs, int64_t sb_stride, void* y,
+                                             int64_t M, int64_t K, int64_t N, int group_size,
+                                             int bits, void* workspace, size_t workspace_bytes,
+                                             void* stream) {
+  if (!sb_pairs || N % 4 || sb_stride < N || sb_stride % 4 || group_size < 32 ||
+      sb_stride > 0xFFFFFFFFll / 4 || sb_stride * (K / group_size) * 4 > 0xFFFFFFFFll) {
+    set_error("dfmi_qmm_affine_pairs_strided: sb_stride %lld needs a pair table, N <= sb_stride, "
+              "N %% 4 == 0, sb_stride %% 4 == 0 and a table under 4 GiB", (long long)sb_stride);
+    return DFMI_EINVAL;
+  }
+  return qmm_affine(x, x_dtype, w_q, scales, biases, sb_pairs, sb_stride, y, M, K, N, group_size,
+                    bits, workspace, workspace_bytes, nullptr, stream);
 }
 
 extern "C" int dfmi_qmm_affine_ex(const void* x, int x_dtype, const uint32_t* w_q,
@@ -1181,6 +1221,11 @@ extern "C" int dfmi_qmm_affine_noalloc(const void* x, int x_dtype, const uint32_
   int rc = validate_qmm(x_dtype, M, K, N, group_size, bits);
   if (rc != DFMI_OK) return rc;
   if (M == 0 || N == 0) return DFMI_OK;
+  // more rows than the streaming kernels take: the general kernel, which
+  // needs no scratch (so such calls may overlap)
+  if (use_gemm(M, K, N, group_size, nullptr))
+    return dfmi_qmm_affine_ex(x, x_dtype, w_q, scales, biases, y, M, K, N, group_size, bits,
+                              nullptr, 0, nullptr, stream);
   const size_t need = dfmi_qmm_workspace_bytes_ex(M, K, N, group_size, bits, nullptr);
   if (need > kScratchBytes) {
     set_error("dfmi_qmm_affine_noalloc: shape M=%lld K=%lld N=%lld needs %zu workspace bytes, "

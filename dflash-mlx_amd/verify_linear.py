@@ -194,7 +194,7 @@ class _VerifyState:
     and the sibling group it belongs to."""
 
     __slots__ = ("w", "s", "b", "N", "K", "gs", "bits", "pairs", "pairs_ok", "stride", "recs",
-                 "group", "gidx")
+                 "group", "gidx", "vers")
 
     def __init__(self, w, s, b, N, K, gs, bits):
         self.w, self.s, self.b = w, s, b
@@ -206,6 +206,19 @@ class _VerifyState:
         self.recs = {}
         self.group = None
         self.gidx = 0
+        self.vers = None
+
+    def current_table(self, obj):
+        """The pair table, if the module's tensors are still the ones it was
+        built from, unchanged (None: not, or a graph is being captured before
+        it exists)."""
+        if not self.pairs_ok or obj.weight is not self.w or obj.scales is not self.s or \
+                obj.biases is not self.b:
+            return None
+        if self.pairs is None and torch.cuda.is_current_stream_capturing():
+            return None
+        t = self.pair_table()
+        return t if self.vers == (self.s._version, self.b._version) else None
 
     def pair_table(self):
         """The pair table (built on first use; None while a graph is being
@@ -217,6 +230,7 @@ class _VerifyState:
                 _warn_capture_without_table()
                 return None
             self.pairs = _runtime.build_sb_pairs(self.s, self.b)
+            self.vers = (self.s._version, self.b._version)
         return self.pairs
 
     def record(self, m: int, st: int, x: torch.Tensor) -> LaunchRecord:
@@ -299,6 +313,12 @@ def _build_dispatch(obj: VerifyQuantizedLinear, *, enable_qmm: Optional[bool] = 
                     if y is None:
                         y = state.launch(x, m, st)
                 y = y.view(*shp[:-1], N)
+            elif (x.dtype == sdt and x.is_cuda and m > 32 and kx == K and mode == "affine"
+                  and (t := state.current_table(obj)) is not None):
+                # many rows: the stock route, with the table the module holds
+                y = qmm_launch(_runtime.aligned_contiguous(x.reshape(m, kx)), state.w, state.s,
+                               state.b, N, gs, bits, pairs=t,
+                               pair_stride=state.stride).view(*shp[:-1], N)
             else:
                 y = _stock(x)
             return y + bias if bias is not None else y

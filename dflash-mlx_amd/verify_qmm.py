@@ -111,7 +111,10 @@ def _pairs_of(M: int, K: int, N: int, group_size: int, bits: int, scales, biases
     """The pair table a launch passes: the given one, else the functional
     cache's for shapes whose plan can use it (None: none)."""
     if pairs is None:
-        if not _runtime.pair_shape(M, K, N, group_size, bits):
+        if _runtime.many_rows(M):
+            if K % group_size or K // group_size * N * 4 > 0xFFFFFFFF:
+                return None
+        elif not _runtime.pair_shape(M, K, N, group_size, bits):
             return None
         pairs = _runtime.PAIRS.get(scales, biases)
     return pairs
@@ -127,18 +130,27 @@ def _pairs_ptr(M: int, K: int, N: int, group_size: int, bits: int, scales, biase
 def qmm_launch(x2: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
                N: int, group_size: int, bits: int, tuning=None,
                out: Optional[torch.Tensor] = None,
-               pairs: Optional[torch.Tensor] = None) -> torch.Tensor:
+               pairs: Optional[torch.Tensor] = None, pair_stride: int = 0) -> torch.Tensor:
     """One ``dfmi_qmm_affine_pairs`` launch on the current stream:
     ``[M, K] -> [M, N]``.  ``pairs`` is the layer's pair table
-    (``_runtime.build_sb_pairs``); when None, the one cached for ``scales`` is
-    used (built on first use).  The result does not depend on it."""
+    (``_runtime.build_sb_pairs``), or its column slice of a wider table of
+    ``pair_stride`` columns; when None, the one cached for ``scales`` is used
+    (built on first use).  The result does not depend on it."""
     lib = _lib.load()
     M, K = int(x2.shape[0]), int(x2.shape[1])
     dev = x2.device
     y = out if out is not None else torch.empty((M, N), dtype=x2.dtype, device=dev)
     tptr = ctypes.byref(tuning) if tuning is not None else None
     need = int(lib.dfmi_qmm_workspace_bytes_ex(M, K, N, int(group_size), int(bits), tptr))
-    ws, ws_bytes = _runtime.workspace(dev, need) if need else (0, 0)
+    space = _runtime.optional_workspace if _runtime.many_rows(M) else _runtime.workspace
+    ws, ws_bytes = space(dev, need) if need else (0, 0)
+    if pair_stride and tuning is None:
+        status = lib.dfmi_qmm_affine_pairs_strided(
+            x2.data_ptr(), _runtime.dtype_code(x2.dtype), w.data_ptr(), scales.data_ptr(),
+            biases.data_ptr(), pairs.data_ptr(), int(pair_stride), y.data_ptr(), M, K, N,
+            int(group_size), int(bits), ws, ws_bytes, _runtime.stream_ptr(dev))
+        _lib.check(status, "dfmi_qmm_affine_pairs_strided")
+        return y
     tp = _pairs_ptr(M, K, N, group_size, bits, scales, biases, pairs)
     status = lib.dfmi_qmm_affine_pairs(
         x2.data_ptr(), _runtime.dtype_code(x2.dtype), w.data_ptr(), scales.data_ptr(),
@@ -174,11 +186,12 @@ def qmm_multi_launch(x2: torch.Tensor, mats, group_size: int, bits: int,
         segs[i].sb_pairs = t.data_ptr() if t is not None else 0
     ns = (ctypes.c_int64 * n)(*Ns)
     need = int(lib.dfmi_qmm_multi_workspace_bytes(M, K, ns, n, int(group_size), int(bits)))
-    ws, ws_bytes = _runtime.workspace(dev, need) if need else (0, 0)
+    space = _runtime.optional_workspace if _runtime.many_rows(M) else _runtime.workspace
+    ws, ws_bytes = space(dev, need) if need else (0, 0)
     # two or three matrices with tables: the tables side by side, so that the
     # fused kernel starts its first loads without reading a segment table
     fused = (_runtime.FUSED_PAIRS.get(tables)
-             if 2 <= n <= 3 and all(t is not None for t in tables) else None)
+             if 2 <= n <= 3 and not _runtime.many_rows(M) and all(t is not None for t in tables) else None)
     if fused is not None:
         status = lib.dfmi_qmm_affine_multi_fused(
             x2.data_ptr(), _runtime.dtype_code(x2.dtype), segs, n, fused.data_ptr(), M, K,
@@ -245,7 +258,8 @@ class LaunchRecord:
             ns = (ctypes.c_int64 * n)(*Ns)
             need = int(lib.dfmi_qmm_multi_workspace_bytes(M, K, ns, n, int(group_size),
                                                           int(bits)))
-        ws, ws_bytes = _runtime.workspace(dev, need) if need else (0, 0)
+        space = _runtime.optional_workspace if _runtime.many_rows(M) else _runtime.workspace
+        ws, ws_bytes = space(dev, need) if need else (0, 0)
         buf = ctypes.create_string_buffer(_lib.DFMI_QMM_RECORD_BYTES + 16)
         ptr = (ctypes.addressof(buf) + 15) // 16 * 16
         status = lib.dfmi_qmm_prepare(_runtime.dtype_code(dtype), segs, n,
@@ -343,7 +357,8 @@ def _general(x, w, scales, biases, transpose: bool, group_size: int, bits: int):
     need = 0
     if transpose and x.dtype == scales.dtype and x.dtype != torch.float32:
         need = int(lib.dfmi_qmm_workspace_bytes(M, K, N, group_size, bits))
-    ws, ws_bytes = _runtime.workspace(x.device, need) if need else (0, 0)
+    space = _runtime.optional_workspace if _runtime.many_rows(M) else _runtime.workspace
+    ws, ws_bytes = space(x.device, need) if need else (0, 0)
     status = lib.dfmi_qmm_general(
         x2.data_ptr(), _runtime.dtype_code(x2.dtype), wq.data_ptr(), s.data_ptr(), b.data_ptr(),
         _runtime.dtype_code(s.dtype), y.data_ptr(), M, K, N, group_size, bits, int(bool(transpose)),

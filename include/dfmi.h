@@ -96,6 +96,10 @@ typedef struct dfmi_qmm_tuning {
  * on scheduling: every K split is summed in a fixed order.  Shapes that split
  * K across workgroups need the workspace dfmi_qmm_workspace_bytes reports
  * (0 bytes -> workspace may be NULL); it must be zero-filled when created.
+ * With more than 32 rows the workspace is optional: the matrix-core kernel
+ * keeps the partial tiles of a K split in it, and the pair table where the
+ * call brings none; with less of it the call runs unsplit, or on the general
+ * kernel (the sums of another split are in another fp32 order).
  */
 int dfmi_qmm_affine(const void *x, int x_dtype, const uint32_t *w_q, const void *scales,
                     const void *biases, void *y, int64_t M, int64_t K, int64_t N,
@@ -146,6 +150,17 @@ int dfmi_qmm_affine_pairs(const void *x, int x_dtype, const uint32_t *w_q, const
                           const void *biases, const uint32_t *sb_pairs, void *y, int64_t M,
                           int64_t K, int64_t N, int group_size, int bits, void *workspace,
                           size_t workspace_bytes, const dfmi_qmm_tuning *tuning, void *stream);
+/*
+ * dfmi_qmm_affine_pairs with the automatic plan, for a matrix whose pair
+ * table is a column slice of a wider one (a sibling group's): sb_pairs points
+ * at the matrix's first column, sb_stride is the wider table's row length.
+ * N and sb_stride are multiples of 4.
+ */
+int dfmi_qmm_affine_pairs_strided(const void *x, int x_dtype, const uint32_t *w_q,
+                                  const void *scales, const void *biases,
+                                  const uint32_t *sb_pairs, int64_t sb_stride, void *y, int64_t M,
+                                  int64_t K, int64_t N, int group_size, int bits, void *workspace,
+                                  size_t workspace_bytes, void *stream);
 /*
  * Pair table for dfmi_qmm_affine_pairs / dfmi_qmm_affine_multi: from scales
  * and biases [N, groups] (dtype DFMI_BF16 or DFMI_F16, the layer's 16-bit
