@@ -106,6 +106,10 @@ _SIGNATURES = {
                                             _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                                             _c_void_p, _i64, _i64, _i64, _i64, _int, _int,
                                             _c_void_p, _size, _c_void_p]),
+    "dfmi_switch_glu_workspace_bytes": (_size, [_i64]),
+    "dfmi_switch_glu": (_int, [_c_void_p, _int, _i64, _c_void_p, _int, _i64] + [_c_void_p] * 13 +
+                        [_i64, _i64, _i64, _int, _int, _c_void_p, _size, _c_void_p, _size,
+                         _c_void_p]),
     "dfmi_gather_qmm_swiglu_pairs": (_int, [_c_void_p, _int, _i64, _c_void_p, _c_void_p,
                                             _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                                             _c_void_p, _c_void_p, _c_void_p, _c_void_p, _i64,

@@ -202,4 +202,18 @@ __device__ inline uint32_t key_index(unsigned long long key) {
   return 0xFFFFFFFFu - (uint32_t)(key & 0xFFFFFFFFull);
 }
 
+template <typename Tag>
+__device__ inline float rnd(float v) {
+  return Num<Tag>::h2f(Num<Tag>::f2h(v));
+}
+
+// silu(g) * u with every op rounded to the activation dtype, as the
+// op-by-op MLX sequence sigmoid(g) -> g * sig -> * u does.
+template <typename Tag>
+__device__ inline float silu_mul(float g, float u) {
+  const float sig = rnd<Tag>(1.0f / (1.0f + __expf(-g)));
+  const float si = rnd<Tag>(g * sig);
+  return si * u;
+}
+
 }  // namespace dfmi

@@ -62,7 +62,8 @@ struct GemmArgs {
   int vec;             // y rows are 16-byte aligned: whole-piece stores
 };
 
-template <typename Tag, int GS, int BITS, int MT, int NT, int WM, int WN>
+// ROWS: the tile's activation rows are given one by one (xr), not consecutive.
+template <typename Tag, int GS, int BITS, int MT, int NT, int WM, int WN, bool ROWS = false>
 struct Gemm {
   static constexpr int WAVES = WM * WN, THREADS = 64 * WAVES;
   static constexpr int BM = 32 * MT * WM, BN = 32 * NT * WN;
@@ -156,12 +157,13 @@ struct Gemm {
     // DMA, first instruction, step 0: this lane's activation row and piece in
     // it, weight piece and pairs, as byte offsets
     uint32_t xg, xp, wg, tg;
+    uint32_t xr[ROWS ? X_DMA : 1];  // ROWS: byte offset of each instruction's row
     uint32_t xo[4];             // activation fragment q of unit 0 in a stage, row block 0
     uint32_t xs[2];             // fragment (k half of unit 0) of 16-row blocks, the wavefront's first
     uint32_t wo[2];             // weight piece e of unit 0 in a stage, column tile 0
     uint32_t to;                // pair of group 0, column tile 0, in a stage
     uint32_t xstride, wstride;  // row bytes
-    int K, groups, wave, wm, wn, lane, h, n0;
+    int K, groups, wave, wm, wn, lane, h;
     uint32_t tn;
     u32x4 ones;
   };
@@ -175,7 +177,10 @@ struct Gemm {
   // swizzle key of a weight row in a stage
   __device__ static inline int wkey(int r) { return BITS == 4 ? (r >> 2) & 3 : r & 7; }
 
-  __device__ static inline void setup(Ctx& cx, const GemmArgs& a, int m0, int n0) {
+  // The lane's constants: K, the pair table's row length, and the first
+  // column and number of columns of the tile in it.  The buffers are the
+  // caller's.
+  __device__ static inline void setup(Ctx& cx, int K, uint32_t tn, int n0, int cols) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     cx.lane = lane;
@@ -183,17 +188,11 @@ struct Gemm {
     cx.wm = wave / WN;
     cx.wn = wave % WN;
     cx.h = lane >> 5;
-    cx.K = a.K;
-    cx.n0 = n0;
-    cx.groups = a.K / GS;
-    cx.tn = a.tn;
-    const int rows = min(BM, a.M - m0), cols = min(BN, a.N - n0);
-    cx.xstride = (uint32_t)a.K * 2u;
-    cx.wstride = (uint32_t)(a.K / 8 * BITS);
-    // the buffers end with the tile's last row: reads past it return zeros
-    cx.x = buffer_rsrc(a.x + (int64_t)m0 * a.K, (uint32_t)rows * cx.xstride);
-    cx.w = buffer_rsrc(a.w + (int64_t)n0 * (cx.wstride / 4), (uint32_t)cols * cx.wstride);
-    cx.t = buffer_rsrc(a.t, a.tn * (uint32_t)cx.groups * 4u);
+    cx.K = K;
+    cx.groups = K / GS;
+    cx.tn = tn;
+    cx.xstride = (uint32_t)K * 2u;
+    cx.wstride = (uint32_t)(K / 8 * BITS);
     // activation DMA: one instruction brings 4 rows; slot s of row r holds
     // piece s ^ (r & 15).  Instruction i of a wavefront is 4 i rows on, which
     // flips bits 2 and 3 of the key
@@ -213,7 +212,7 @@ struct Gemm {
     {
       const int o = wave * TPB + 16 * lane;
       const int grp = o / (4 * BN), row = (o % (4 * BN)) / 4;
-      cx.tg = (lane < TLANES && row < cols) ? ((uint32_t)grp * a.tn + (uint32_t)(n0 + row)) * 4u
+      cx.tg = (lane < TLANES && row < cols) ? ((uint32_t)grp * tn + (uint32_t)(n0 + row)) * 4u
                                             : kNoRow;
     }
     // fragments
@@ -263,7 +262,8 @@ struct Gemm {
 #pragma unroll
     for (int i = 0; i < X_DMA; ++i) {
       const uint32_t piece = cx.xp ^ (uint32_t)(64 * (i & 3));
-      uint32_t off = piece + (cx.xg + (uint32_t)(4 * i) * cx.xstride);
+      uint32_t off =
+          piece + (ROWS ? cx.xr[ROWS ? i : 0] : cx.xg + (uint32_t)(4 * i) * cx.xstride);
       if (PART && (int)piece >= 2 * left) off = kNoRow;
       dma16(cx.x, off, (uint32_t)c * (uint32_t)XROW, base + (cx.wave * X_DMA + i) * 1024);
     }
@@ -596,7 +596,12 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qmm_gemm_kernel(GemmArgs a) {
   const int c0 = (int)((int64_t)kpi * a.steps / a.kp);
   const int c1 = (int)((int64_t)(kpi + 1) * a.steps / a.kp);
   typename G::Ctx cx;
-  G::setup(cx, a, m0, n0);
+  const int rows = min(G::BM, a.M - m0), cols = min(G::BN, a.N - n0);
+  G::setup(cx, a.K, a.tn, n0, cols);
+  // the buffers end with the tile's last row: reads past it return zeros
+  cx.x = buffer_rsrc(a.x + (int64_t)m0 * a.K, (uint32_t)rows * cx.xstride);
+  cx.w = buffer_rsrc(a.w + (int64_t)n0 * (cx.wstride / 4), (uint32_t)cols * cx.wstride);
+  cx.t = buffer_rsrc(a.t, a.tn * (uint32_t)cx.groups * 4u);
   typename G::Acc acc;
 #pragma unroll
   for (int i = 0; i < MT; ++i)

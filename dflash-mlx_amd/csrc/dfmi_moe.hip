@@ -22,6 +22,7 @@
 
 #include "dfmi_core.h"
 #include "dfmi_host.h"
+#include "dfmi_moe_gemm.h"
 #include "dfmi_stream.h"
 
 namespace dfmi {
@@ -40,21 +41,16 @@ struct GatherArgs {
   uint16_t* y;           // [P, N]
   int P, K, N, E;
   int chunks;
+  // > 0: lhs holds pair ids; pair p reads activation row lhs[p] / div and
+  // writes output row lhs[p] (expert-sorted pairs, results in pair order)
+  int div;
+
+  __device__ inline int x_row(int p) const {
+    const int l = lhs ? lhs[p] : p;
+    return div > 1 ? l / div : l;
+  }
+  __device__ inline int64_t y_row(int p) const { return div > 0 ? lhs[p] : p; }
 };
-
-template <typename Tag>
-__device__ inline float rnd(float v) {
-  return Num<Tag>::h2f(Num<Tag>::f2h(v));
-}
-
-// silu(g) * u with every op rounded to the activation dtype, as the
-// op-by-op MLX sequence sigmoid(g) -> g * sig -> * u does.
-template <typename Tag>
-__device__ inline float silu_mul(float g, float u) {
-  const float sig = rnd<Tag>(1.0f / (1.0f + __expf(-g)));
-  const float si = rnd<Tag>(g * sig);
-  return si * u;
-}
 
 template <typename Tag, int GS, int NT, bool KFULL, bool GLU>
 __global__ __launch_bounds__(kMaxWaves * 64) void gather_kernel(GatherArgs a) {
@@ -94,7 +90,7 @@ __global__ __launch_bounds__(kMaxWaves * 64) void gather_kernel(GatherArgs a) {
     const int rows = min(16, run - g0);
     // activation row of this lane's MFMA row (rows past the run repeat the last pair)
     const int pl = p + g0 + min(lane & 15, rows - 1);
-    int xr_row = a.lhs ? a.lhs[pl] : pl;
+    int xr_row = a.x_row(pl);
     if (xr_row < 0 || xr_row >= a.x_rows) xr_row = 0;  // reported as NaN below
     typename C::XRows xr;
     xr.off[0] = (int64_t)xr_row * a.K;
@@ -128,7 +124,7 @@ __global__ __launch_bounds__(kMaxWaves * 64) void gather_kernel(GatherArgs a) {
       const int n = n0 + t * 16 + (l & 15);
       if (m < rows && n < a.N) {
         const int pp = p + g0 + m;
-        const int xrow = a.lhs ? a.lhs[pp] : pp;
+        const int xrow = a.x_row(pp);
         float out;
         if (bad_e || xrow < 0 || xrow >= a.x_rows) {
           out = __builtin_nanf("");
@@ -137,7 +133,7 @@ __global__ __launch_bounds__(kMaxWaves * 64) void gather_kernel(GatherArgs a) {
         } else {
           out = v;
         }
-        a.y[(int64_t)pp * a.N + n] = Num<Tag>::f2h(out);
+        a.y[a.y_row(pp) * a.N + n] = Num<Tag>::f2h(out);
       }
     }
     __syncthreads();  // the next group reuses the reduction buffer
@@ -160,7 +156,7 @@ __global__ __launch_bounds__(256) void gather_stream_kernel(GatherArgs a) {
     s_rhs[tid] = (q >= 0 && q < a.P) ? a.rhs[q] : 0;
   } else if (tid >= 64 && tid < 80) {
     const int q = min(p + tid - 64, a.P - 1);
-    s_lhs[tid - 64] = a.lhs ? a.lhs[q] : q;
+    s_lhs[tid - 64] = a.x_row(q);
   }
   __syncthreads();
   const int e = s_rhs[1];
@@ -196,7 +192,7 @@ __global__ __launch_bounds__(256) void gather_stream_kernel(GatherArgs a) {
     const int rows = min(16, run - g0);
     if (g0 > 0 && tid < 16) {  // later row blocks of a long run
       const int pp = p + g0 + min(tid, rows - 1);
-      s_lhs[tid] = a.lhs ? a.lhs[pp] : pp;
+      s_lhs[tid] = a.x_row(pp);
     }
     __syncthreads();
     if (tid < 16) {
@@ -244,7 +240,7 @@ __global__ __launch_bounds__(256) void gather_stream_kernel(GatherArgs a) {
         } else {
           out = v;
         }
-        a.y[(int64_t)pp * a.N + n] = Num<Tag>::f2h(out);
+        a.y[a.y_row(pp) * a.N + n] = Num<Tag>::f2h(out);
       }
     }
     __syncthreads();  // s_lhs, s_rows and the LDS stages are reused by the next row block
@@ -331,13 +327,13 @@ __global__ __launch_bounds__(512) void gather_persist_kernel(GatherArgs a) {
   const int32_t* const alhs = a.lhs;
   const int32_t* const arhs = a.rhs;
   uint16_t* const ay = a.y;
-  const int K = a.K, N = a.N, E = a.E;
+  const int K = a.K, N = a.N, E = a.E, div = a.div;
 
   // --- segment table: pairs -> runs of one expert -> segments of <= 16 pairs
   for (int i = tid; i < P; i += 512) {
-    const int l = alhs ? alhs[i] : i;
+    const int id = alhs ? alhs[i] : i, l = div > 1 ? id / div : id;
     t_rhs[i] = arhs[i];
-    t_lhs[i] = l;
+    t_lhs[i] = id;
     t_xr[i] = (l < 0 || l >= x_rows) ? 0 : l;  // invalid rows read row 0, reported as NaN
   }
   __syncthreads();
@@ -525,7 +521,7 @@ __global__ __launch_bounds__(512) void gather_persist_kernel(GatherArgs a) {
       const int l = el & 63, jj = (el >> 6) & 3, t = el >> 8;
       const int m = 4 * (l >> 4) + jj;
       const int n = n0 + 16 * t + (l & 15);
-      const int xrow = t_lhs[p0 + min(m, rows - 1)];
+      const int id = t_lhs[p0 + min(m, rows - 1)], xrow = div > 1 ? id / div : id;
       float out;
       if (bad_e || xrow < 0 || xrow >= x_rows) {
         out = __builtin_nanf("");
@@ -534,8 +530,8 @@ __global__ __launch_bounds__(512) void gather_persist_kernel(GatherArgs a) {
       } else {
         out = v;
       }
-      const uint32_t off =
-          (m < rows && n < N) ? (uint32_t)(((int64_t)(p0 + m) * N + n) * 2) : kNoRow;
+      const int64_t yrow = div > 0 ? id : p0 + m;
+      const uint32_t off = (m < rows && n < N) ? (uint32_t)((yrow * N + n) * 2) : kNoRow;
       __builtin_amdgcn_raw_buffer_store_b16(Num<Tag>::f2h(out), yr, off, 0, 0);
     }
   };
@@ -616,7 +612,8 @@ struct MoeLayout {
   static constexpr int SEGE = SEGS + 2 * (kMoeMaxPairs + 2);   // u16[P]: segment expert
   static constexpr int NSEG = SEGE + 2 * kMoeMaxPairs;
   static constexpr int FLAG = NSEG + 4;  // int: this workgroup's piece completed its unit
-  static constexpr int BYTES = FLAG + 4;
+  static constexpr int YR = FLAG + 4;    // u8[P]: output row (< P)
+  static constexpr int BYTES = YR + kMoeMaxPairs;
   static_assert(BYTES <= 80 * 1024, "two workgroups per CU");
   static_assert(RUNM % 8 == 0 && NSEG % 4 == 0, "alignment");
 };
@@ -628,8 +625,10 @@ struct MoeLayout {
 template <typename Tag, int GS, bool GLU>
 __global__ __launch_bounds__(512) void moe_stream_kernel(
     const int32_t* g_lhs, const int32_t* g_rhs, const uint16_t* g_x, const uint32_t* g_w0,
-    const uint32_t* g_w1, const uint32_t* g_t, int g_P, int g_K, int g_N, int g_E,
+    const uint32_t* g_w1, const uint32_t* g_t, int g_Pd, int g_K, int g_N, int g_E,
     int64_t g_x_rows, uint16_t* g_y, uint32_t* g_wsc, float* g_wsp) {
+  // P and GatherArgs::div in one of the preloaded argument words
+  const int g_P = g_Pd & 0xFFFF, div = (int)((uint32_t)g_Pd >> 16);
   GatherArgs a;
   a.x = g_x;
   a.x_rows = g_x_rows;
@@ -648,6 +647,7 @@ __global__ __launch_bounds__(512) void moe_stream_kernel(
   a.N = g_N;
   a.E = g_E;
   a.chunks = 0;
+  a.div = div;
   using LY = MoeLayout<Tag, GS>;
   using S = typename LY::S;
   constexpr int OUTC = GLU ? 64 : 128;  // output columns per unit
@@ -658,6 +658,7 @@ __global__ __launch_bounds__(512) void moe_stream_kernel(
   uint64_t* t_run = reinterpret_cast<uint64_t*>(dfmi_smem + LY::RUNM);
   uint64_t* t_segm = reinterpret_cast<uint64_t*>(dfmi_smem + LY::SEGM);
   uint16_t* t_xr = reinterpret_cast<uint16_t*>(dfmi_smem + LY::XR);
+  uint8_t* t_yr = reinterpret_cast<uint8_t*>(dfmi_smem + LY::YR);
   uint16_t* t_seg = reinterpret_cast<uint16_t*>(dfmi_smem + LY::SEGS);
   uint16_t* t_se = reinterpret_cast<uint16_t*>(dfmi_smem + LY::SEGE);
   int* t_nseg = reinterpret_cast<int*>(dfmi_smem + LY::NSEG);
@@ -681,8 +682,9 @@ __global__ __launch_bounds__(512) void moe_stream_kernel(
   int e_p = 0;
   bool st = false;  // pair tid starts a run
   if (tid < P) {
-    const int l = alhs ? alhs[tid] : tid;
+    const int id = alhs ? alhs[tid] : tid, l = div > 1 ? id / div : id;
     t_xr[tid] = (uint16_t)((l < 0 || l >= x_rows) ? 0x8000 : l);
+    t_yr[tid] = (uint8_t)(div > 0 ? id : tid);
     e_p = arhs[tid];
     st = tid == 0 || e_p != arhs[tid - 1];
   }
@@ -989,8 +991,8 @@ __global__ __launch_bounds__(512) void moe_stream_kernel(
         } else {
           out = g[q];
         }
-        const uint32_t off =
-            m < rows ? (uint32_t)(((int64_t)(p0 + m) * N + n) * 2) : kNoRow;
+        const int yrow = t_yr[p0 + min(m, rows - 1)];
+        const uint32_t off = m < rows ? (uint32_t)(((int64_t)yrow * N + n) * 2) : kNoRow;
         __builtin_amdgcn_raw_buffer_store_b16(Num<Tag>::f2h(out), yr, off, 0, 0);
       }
     }
@@ -1034,7 +1036,8 @@ static void launch_moe_stream_t(const GatherArgs& a, int grid, hipStream_t st) {
       hipFuncAttributeMaxDynamicSharedMemorySize, LY::BYTES);
   (void)attr;
   hipLaunchKernelGGL((moe_stream_kernel<Tag, GS, GLU>), dim3(grid), dim3(512), LY::BYTES, st,
-                     a.lhs, a.rhs, a.x, a.w[0], a.w[1], a.t, a.P, a.K, a.N, a.E, a.x_rows, a.y,
+                     a.lhs, a.rhs, a.x, a.w[0], a.w[1], a.t,
+                     (int)((uint32_t)a.P | ((uint32_t)a.div << 16)), a.K, a.N, a.E, a.x_rows, a.y,
                      a.ws_counters, a.ws_partials);
 }
 
@@ -1164,7 +1167,8 @@ static int gather_common(const void* x, int x_dtype, int64_t x_rows, const uint3
                          const void* b1, const int32_t* lhs_rows, const int32_t* rhs_experts,
                          void* y, int64_t P, int64_t K, int64_t N, int64_t E, int group_size,
                          int bits, bool glu, const uint32_t* pairs, void* workspace,
-                         size_t workspace_bytes, void* stream) {
+                         size_t workspace_bytes, void* stream, int div = 0,
+                         const int32_t* segs = nullptr) {
   int rc = validate_gather(x_dtype, x_rows, P, K, N, E, group_size, bits);
   if (rc != DFMI_OK) return rc;
   if (P == 0 || N == 0) return DFMI_OK;
@@ -1195,6 +1199,7 @@ static int gather_common(const void* x, int x_dtype, int64_t x_rows, const uint3
   a.E = (int)E;
   a.chunks = (int)((K + kChunkK - 1) / kChunkK);
   a.t = pairs;
+  a.div = div;
   const bool ws_ok = workspace && workspace_bytes >= kMoeWsBytes && aligned16(workspace);
   a.ws_counters = ws_ok ? static_cast<uint32_t*>(workspace) : nullptr;
   a.ws_partials =
@@ -1214,6 +1219,35 @@ static int gather_common(const void* x, int x_dtype, int64_t x_rows, const uint3
       else launch_moe_stream<F16, false>(a, group_size, grid, st);
     }
     return check_launch(glu ? "dfmi_gather_qmm_swiglu" : "dfmi_gather_qmm_affine");
+  }
+  // more pairs than that kernel's tables hold: 32-row tiles on the large
+  // matrix instructions, the segment table in the workspace
+  if (pairs && aligned16(pairs) && (segs || ws_ok) &&
+      moe_gemm_eligible(x_rows, P, K, N, E, group_size, glu)) {
+    if (!segs) {
+      int32_t* t = static_cast<int32_t*>(workspace) + kMoeWsCounterBytes / 4;
+      static_assert(kMoeWsBytes - kMoeWsCounterBytes >= 4 * (65535 + 2), "segment table");
+      rc = moe_segments_launch(rhs_experts, (int)P, t, st);
+      if (rc != DFMI_OK) return rc;
+      segs = t;
+    }
+    MoeGemmArgs g{};
+    g.x = a.x;
+    g.w[0] = a.w[0];
+    g.w[1] = a.w[1];
+    g.t = pairs;
+    g.lhs = lhs_rows;
+    g.rhs = rhs_experts;
+    g.segs = segs;
+    g.y = a.y;
+    g.x_rows = x_rows;
+    g.P = (int)P;
+    g.K = (int)K;
+    g.N = (int)N;
+    g.E = (int)E;
+    g.div = div;
+    g.vec = aligned16(y);
+    return moe_gemm_launch(g, x_dtype, group_size, glu, st);
   }
   // persistent pipelined loop: whole 512-k steps, a full-K scale window of
   // at most 4 pieces, the pair tables in LDS, 32-bit buffer offsets.
@@ -1395,6 +1429,54 @@ extern "C" int dfmi_gather_qmm_swiglu_pairs(const void* x, int x_dtype, int64_t 
   return gather_common(x, x_dtype, x_rows, wg_q, g_scales, g_biases, wu_q, u_scales, u_biases,
                        lhs_rows, rhs_experts, h, P, K, N, E, group_size, bits, true, sb_pairs,
                        workspace, workspace_bytes, stream);
+}
+
+// Workspace of dfmi_switch_glu: the pair ids and experts in expert order and
+// the segment table.
+static size_t switch_glu_ints(int64_t P) { return (size_t)((P + 63) / 64 * 64); }
+
+extern "C" size_t dfmi_switch_glu_workspace_bytes(int64_t P) {
+  return P > 0 && P <= 65535 ? (3 * switch_glu_ints(P) + 64) * 4 : 0;
+}
+
+extern "C" int dfmi_switch_glu(const void* x, int x_dtype, int64_t T, const void* inds,
+                               int inds_bytes, int64_t k, const uint32_t* wg_q,
+                               const void* g_scales, const void* g_biases, const uint32_t* wu_q,
+                               const void* u_scales, const void* u_biases, const uint32_t* wd_q,
+                               const void* d_scales, const void* d_biases,
+                               const uint32_t* glu_pairs, const uint32_t* down_pairs, void* h,
+                               void* y, int64_t D, int64_t I, int64_t E, int group_size, int bits,
+                               void* workspace, size_t workspace_bytes, void* gather_workspace,
+                               size_t gather_workspace_bytes, void* stream) {
+  if (T < 0 || k < 1 || k > 65535 || T > 65535 || (inds_bytes != 4 && inds_bytes != 8) ||
+      E > kMoeSortMaxExperts) {
+    set_error("dfmi_switch_glu: bad arguments T=%lld k=%lld E=%lld, %d-byte expert ids",
+              (long long)T, (long long)k, (long long)E, inds_bytes);
+    return DFMI_EINVAL;
+  }
+  const int64_t P = T * k;
+  int rc = validate_gather(x_dtype, T, P, D, I, E, group_size, bits);
+  if (rc == DFMI_OK) rc = validate_gather(x_dtype, P, P, I, D, E, group_size, bits);
+  if (rc != DFMI_OK || P == 0) return rc;
+  if (!inds || !workspace || !aligned16(workspace) ||
+      workspace_bytes < dfmi_switch_glu_workspace_bytes(P)) {
+    set_error("dfmi_switch_glu: expert ids and a workspace of %zu bytes (16-byte aligned) required",
+              dfmi_switch_glu_workspace_bytes(P));
+    return inds ? DFMI_ENOSPC : DFMI_EINVAL;
+  }
+  int32_t* order = static_cast<int32_t*>(workspace);
+  int32_t* rhs = order + switch_glu_ints(P);
+  int32_t* segs = rhs + switch_glu_ints(P);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  rc = moe_sort_launch(inds, inds_bytes, (int)P, (int)E, order, rhs, segs, st);
+  if (rc != DFMI_OK) return rc;
+  rc = gather_common(x, x_dtype, T, wg_q, g_scales, g_biases, wu_q, u_scales, u_biases, order, rhs,
+                     h, P, D, I, E, group_size, bits, true, glu_pairs, gather_workspace,
+                     gather_workspace_bytes, stream, (int)k, segs);
+  if (rc != DFMI_OK) return rc;
+  return gather_common(h, x_dtype, P, wd_q, d_scales, d_biases, nullptr, nullptr, nullptr, order,
+                       rhs, y, P, I, D, E, group_size, bits, false, down_pairs, gather_workspace,
+                       gather_workspace_bytes, stream, 1, segs);
 }
 
 // Pair tables of expert weights: [E][G][N] from one (scales, biases) set, or

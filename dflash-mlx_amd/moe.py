@@ -18,7 +18,7 @@ the gate/up pair plus SwiGLU is one ``dfmi_gather_qmm_swiglu`` launch (one
 pass over both weight sets), and the weighted sum is ``dfmi_moe_combine``.
 
 Where the expert shapes allow (4-bit, gs 64 / 128, K a multiple of 256,
-N a multiple of 128, or 64 for the SwiGLU pair, at most 256 pairs) the
+N a multiple of 128, or 64 for the SwiGLU pair) the
 gathers take the experts' (scale, bias) pair table (``dfmi_moe_pairs``,
 built once per weight set and cached) and the stream's gather workspace, and
 run the pair-streaming main loop (``dfmi_gather_qmm_*_pairs``); otherwise,
@@ -187,6 +187,46 @@ def moe_combine(y: torch.Tensor, scores: torch.Tensor, *,
     return out
 
 
+_SORT_MAX_EXPERTS = 1023  # of dfmi_switch_glu
+
+
+def _switch_glu(x, inds, gate: Triple, up: Triple, down: Triple, group_size: int, bits: int):
+    """``dfmi_switch_glu``: sort, both gathers and the pair order in one call.
+    None where it does not apply: x or down of other shapes than one layer's,
+    or a graph capture before the stream has the workspaces."""
+    _runtime.require_device(x, "x")
+    dev = x.device
+    T, k = int(inds.shape[0]), int(inds.shape[1])
+    D = int(x.shape[-1])
+    x2 = _runtime.aligned_contiguous(x.reshape(-1, D))
+    E, I, wg, sg, bg = _expert_weights(*gate, D, group_size, bits)
+    Eu, Iu, wu, su, bu = _expert_weights(*up, D, group_size, bits)
+    if (E, I) != (Eu, Iu):
+        raise ValueError("gate and up expert weights must have the same [E, N]")
+    Ed, Nd, wd, sd, bd = _expert_weights(*down, I, group_size, bits)
+    if int(x2.shape[0]) != T or (Ed, Nd) != (E, D):
+        return None
+    ids = inds.contiguous()
+    P = T * k
+    lib = _lib.load()
+    need = int(lib.dfmi_switch_glu_workspace_bytes(P))
+    ws, ws_bytes = _runtime.optional_workspace(dev, need, kind="moe_sort")
+    if ws_bytes < need:
+        return None
+    h = torch.empty((P, I), dtype=x.dtype, device=dev)
+    y = torch.empty((P, D), dtype=x.dtype, device=dev)
+    tg = _pairs_ptr(None, sg, bg, (su, bu), D, I, group_size, bits, True)
+    td = _pairs_ptr(None, sd, bd, None, I, D, group_size, bits, True)
+    gws, gws_bytes = _workspace(lib, dev, tg or td)
+    _lib.check(lib.dfmi_switch_glu(
+        x2.data_ptr(), _runtime.dtype_code(x.dtype), T, ids.data_ptr(), ids.element_size(), k,
+        wg.data_ptr(), sg.data_ptr(), bg.data_ptr(), wu.data_ptr(), su.data_ptr(), bu.data_ptr(),
+        wd.data_ptr(), sd.data_ptr(), bd.data_ptr(), tg, td, h.data_ptr(), y.data_ptr(), D, I, E,
+        int(group_size), int(bits), ws, ws_bytes, gws, gws_bytes, _runtime.stream_ptr(dev)),
+        "dfmi_switch_glu")
+    return h, y
+
+
 def switch_glu(x: torch.Tensor, inds: torch.Tensor, gate: Triple, up: Triple, down: Triple, *,
                group_size: int = 64, bits: int = 4) -> Tuple[torch.Tensor, torch.Tensor]:
     """Per-pair SwitchGLU for ``x`` ``[T, D]`` and expert ids ``inds``
@@ -194,6 +234,12 @@ def switch_glu(x: torch.Tensor, inds: torch.Tensor, gate: Triple, up: Triple, do
     Pairs are sorted by expert (as mlx-lm does) so each expert's weights are
     streamed once, and the results are returned in pair order."""
     T, k = int(inds.shape[0]), int(inds.shape[1])
+    E = int(gate[0].shape[0])
+    if E <= _SORT_MAX_EXPERTS and 0 < T * k <= 65535 and inds.is_cuda and \
+            inds.dtype in (torch.int32, torch.int64):
+        out = _switch_glu(x, inds, gate, up, down, group_size, bits)
+        if out is not None:
+            return out
     flat = inds.reshape(-1).to(torch.int64)
     order = torch.argsort(flat, stable=True)
     rhs = flat[order].to(torch.int32)

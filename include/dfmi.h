@@ -374,6 +374,30 @@ int dfmi_gather_qmm_swiglu_pairs(const void *x, int x_dtype, int64_t x_rows,
                                  const int32_t *rhs_experts, void *h, int64_t P, int64_t K,
                                  int64_t N, int64_t E, int group_size, int bits,
                                  void *workspace, size_t workspace_bytes, void *stream);
+/*
+ * A whole SwitchGLU over the pairs p = t k + j: the pairs are sorted by
+ * expert on the device (stable; ids outside [0, E) give NaN rows), then
+ * dfmi_gather_qmm_swiglu_pairs and dfmi_gather_qmm_affine_pairs run on the
+ * sorted pairs and write their results back in pair order:
+ *   h[p, I] = silu(x[t] . gate[e_p]^T) * (x[t] . up[e_p]^T)
+ *   y[p, D] = h[p] . down[e_p]^T,   e_p = inds[t, j]
+ * Replaces the argsort, the gathers of expert ids and rows, and the unsort
+ * mlx-lm's SwitchGLU wraps around mx.gather_qmm (reached from
+ * engine/target_qwen_gdn.py:865,874).  inds: int32 or int64 (inds_bytes 4 or
+ * 8) [T, k]; glu_pairs / down_pairs: the experts' pair tables or NULL;
+ * workspace: dfmi_switch_glu_workspace_bytes(T k) bytes, contents free;
+ * gather_workspace as for the gathers.  E at most 1023, T k at most 65535.
+ */
+size_t dfmi_switch_glu_workspace_bytes(int64_t P);
+int dfmi_switch_glu(const void *x, int x_dtype, int64_t T, const void *inds, int inds_bytes,
+                    int64_t k, const uint32_t *wg_q, const void *g_scales, const void *g_biases,
+                    const uint32_t *wu_q, const void *u_scales, const void *u_biases,
+                    const uint32_t *wd_q, const void *d_scales, const void *d_biases,
+                    const uint32_t *glu_pairs, const uint32_t *down_pairs, void *h, void *y,
+                    int64_t D, int64_t I, int64_t E, int group_size, int bits, void *workspace,
+                    size_t workspace_bytes, void *gather_workspace,
+                    size_t gather_workspace_bytes, void *stream);
+
 size_t dfmi_gather_workspace_bytes(void);
 
 /*
