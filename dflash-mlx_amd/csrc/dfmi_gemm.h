@@ -526,17 +526,29 @@ struct Gemm {
     st = nst;
   }
 
+  // Request the first stages of steps [c0, c1) (LDS stages free).
+  __device__ static inline void start(const Ctx& cx, int c0, int c1) {
+#pragma unroll
+    for (int k = 0; k < DEPTH; ++k) {
+      if (k < c1 - c0) issue(cx, c0 + k, k * STAGE);
+    }
+  }
+
+  // Accumulate steps [c0, c1), whose first stages start() has requested.  On
+  // return every wavefront is past its last read of the stages; the group
+  // sums' exchange is read until the caller's next barrier.
   __device__ static inline void run(const Ctx& cx, int c0, int c1, Acc& acc) {
+    run(cx, c0, c1, acc, [] {});
+  }
+  // between: called once the stages are free, before the last bias terms.
+  template <typename F>
+  __device__ static inline void run(const Ctx& cx, int c0, int c1, Acc& acc, F&& between) {
     const int n = c1 - c0;
     uint32_t rb[NT][SUB];
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
       for (int s = 0; s < SUB; ++s) rb[j][s] = 0u;
-#pragma unroll
-    for (int k = 0; k < DEPTH; ++k) {
-      if (k < n) issue(cx, c0 + k, k * STAGE);
-    }
     for (int o = threadIdx.x * 16; o < XT; o += THREADS * 16)  // what the first flush reads
       *reinterpret_cast<u32x4*>(dfmi_smem + XT_OFF + XT + o) = u32x4{0u, 0u, 0u, 0u};
     // step 0 in LDS: the later ones may be in flight
@@ -575,6 +587,7 @@ struct Gemm {
       for (int e = 0; e < 16; ++e)
         acc.v[MT - 1][NT - 1][e] = __builtin_fmaf(z.ps[s], z.p[s][e], acc.v[MT - 1][NT - 1][e]);
     stage_barrier<0>();
+    between();
     flush(cx, bp ^ 1, rb, acc, odd);
   }
 };
@@ -607,6 +620,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qmm_gemm_kernel(GemmArgs a) {
   for (int i = 0; i < MT; ++i)
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc.v[i][j] = G::zero16();
+  G::start(cx, c0, c1);
   G::run(cx, c0, c1, acc);
 
   const int h = cx.h, col = cx.wn * 32 * NT + (cx.lane & 31), row = cx.wm * 32 * MT;
