@@ -14,6 +14,8 @@ import torch
 
 from . import _lib
 
+_raw_stream = torch._C._cuda_getCurrentRawStream
+
 _DTYPE_CODES = {
     torch.bfloat16: _lib.DFMI_BF16,
     torch.float16: _lib.DFMI_F16,
@@ -179,18 +181,53 @@ def build_moe_pairs(scales: torch.Tensor, biases: torch.Tensor,
     return pairs
 
 
+def versions(tensors) -> Optional[tuple]:
+    """What shows whether the tensors still hold what they held: each one's
+    version and address (None: inference tensors count no versions)."""
+    try:
+        return tuple([(t._version, t.data_ptr()) for t in tensors])
+    except RuntimeError:
+        return None
+
+
+class _Built:
+    """A table and when it is there: a call on another stream than the one
+    that builds it waits for it on the device.  (During capture nothing is
+    waited for: a capture begins behind a synchronised device.)"""
+
+    __slots__ = ("table", "device", "stream", "event")
+
+    def __init__(self, table: torch.Tensor):
+        self.table = table
+        self.device = table.get_device()
+        self.stream = _raw_stream(self.device)
+        self.event = torch.cuda.Event()
+        self.event.record(torch.cuda.current_stream(self.device))
+
+    def get(self) -> torch.Tensor:
+        event = self.event
+        if (event is not None and _raw_stream(self.device) != self.stream
+                and not torch.cuda.is_current_stream_capturing()):
+            if event.query():
+                self.event = None
+            else:
+                torch.cuda.current_stream(self.device).wait_event(event)
+        return self.table
+
+
 class _PairCache:
     """Pair tables of the (scales, biases) tensors the functional operators
     see, built on first use and kept while the tensors live.  An entry is
     valid only for the same tensor objects at the same versions (an in-place
-    update rebuilds it).  Nothing is built during graph capture: the caller
+    update or storage swapped in rebuilds it; inference tensors count no
+    versions and get no table).  Nothing is built during graph capture: the caller
     then runs without a table (dense matmuls: the same plan, bit-identical
     result; gathers: the plain gather's main loop).  ``experts`` selects the
     routed-expert layout (``dfmi_moe_pairs``; with ``up`` the SwiGLU
     interleave of two sets)."""
 
     def __init__(self):
-        self._lock = threading.Lock()
+        self._lock = threading.RLock()  # (a collection inside may call _drop)
         self._entries: dict[tuple, tuple] = {}
 
     def _drop(self, key: tuple):
@@ -201,13 +238,15 @@ class _PairCache:
             up: Optional[Tuple[torch.Tensor, torch.Tensor]] = None, *, experts: bool = False):
         tensors = (scales, biases) + (tuple(up) if up is not None else ())
         key = (id(scales), id(up[0]) if up is not None else 0, bool(experts))
-        ver = tuple(t._version for t in tensors)
+        ver = versions(tensors)
+        if ver is None:
+            return None
         with self._lock:
             ent = self._entries.get(key)
         if ent is not None:
-            refs, ever, pairs = ent
+            refs, ever, built = ent
             if ever == ver and all(r() is t for r, t in zip(refs, tensors)):
-                return pairs
+                return built.get()
         if torch.cuda.is_current_stream_capturing():
             return None
         if experts:
@@ -215,8 +254,9 @@ class _PairCache:
         else:
             pairs = build_sb_pairs(scales, biases)
         refs = tuple(weakref.ref(t, lambda _r, k=key: self._drop(k)) for t in tensors)
+        built = _Built(pairs)
         with self._lock:
-            self._entries[key] = (refs, ver, pairs)
+            self._entries[key] = (refs, ver, built)
         return pairs
 
 
@@ -231,7 +271,7 @@ class _FusedPairCache:
     launches with the per-matrix tables: the same sums)."""
 
     def __init__(self):
-        self._lock = threading.Lock()
+        self._lock = threading.RLock()  # (a collection inside may call _drop)
         self._entries: dict[tuple, tuple] = {}
 
     def _drop(self, key: tuple):
@@ -240,19 +280,22 @@ class _FusedPairCache:
 
     def get(self, tables) -> Optional[torch.Tensor]:
         key = tuple(id(t) for t in tables)
-        ver = tuple(t._version for t in tables)
+        ver = versions(tables)
+        if ver is None:
+            return None
         with self._lock:
             ent = self._entries.get(key)
         if ent is not None:
-            refs, ever, fused = ent
+            refs, ever, built = ent
             if ever == ver and all(r() is t for r, t in zip(refs, tables)):
-                return fused
+                return built.get()
         if torch.cuda.is_current_stream_capturing():
             return None
         fused = torch.cat(list(tables), dim=1).contiguous()
         refs = tuple(weakref.ref(t, lambda _r, k=key: self._drop(k)) for t in tables)
+        built = _Built(fused)
         with self._lock:
-            self._entries[key] = (refs, ver, fused)
+            self._entries[key] = (refs, ver, built)
         return fused
 
 

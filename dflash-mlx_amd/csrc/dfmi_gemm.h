@@ -49,18 +49,28 @@ typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
 
 constexpr int kGemmK = 128;      // k per step
 
+constexpr int kGemmMaxSeg = 3;   // matrices of one launch
+
+// One or more matrices over the same activations; matrix i's column tiles are
+// tile0 .. of the launch's tiles_n.
 struct GemmArgs {
   const uint16_t* x;
-  const uint32_t* w;
-  const uint32_t* t;  // (scale, bias) pairs [K/GS][tn], the matrix's column 0 first
-  uint16_t* y;
-  float* partials;     // split K: [tile][split][BM x BN] in register order
-  int M, K, N;
-  uint32_t tn;
-  int steps;           // ceil(K / 128)
+  float* partials;    // split K: [tile][split][BM x BN] in register order
+  const uint32_t* w[kGemmMaxSeg];
+  const uint32_t* t[kGemmMaxSeg];  // (scale, bias) pairs [K/GS][tn], the matrix's column 0 first
+  uint16_t* y[kGemmMaxSeg];
+  int N[kGemmMaxSeg], tile0[kGemmMaxSeg];
+  uint32_t tn[kGemmMaxSeg];
+  int nseg, M, K;
+  int steps;  // ceil(K / 128)
   int tiles_m, tiles_n, kp;
-  int vec;             // y rows are 16-byte aligned: whole-piece stores
+  int vec;    // every y's rows are 16-byte aligned: whole-piece stores
 };
+
+// the matrix of column tile nb
+__device__ inline int gemm_seg(const GemmArgs& a, int nb) {
+  return a.nseg > 2 && nb >= a.tile0[2] ? 2 : (a.nseg > 1 && nb >= a.tile0[1] ? 1 : 0);
+}
 
 // ROWS: the tile's activation rows are given one by one (xr), not consecutive.
 template <typename Tag, int GS, int BITS, int MT, int NT, int WM, int WN, bool ROWS = false>
@@ -605,16 +615,23 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qmm_gemm_kernel(GemmArgs a) {
   const int nb = id / (a.kp * a.tiles_m);
   const int rest = id - nb * (a.kp * a.tiles_m);
   const int kpi = rest / a.tiles_m, mb = rest - kpi * a.tiles_m;
-  const int m0 = mb * G::BM, n0 = nb * G::BN;
+  const int g = gemm_seg(a, nb);
+  const uint32_t* const w = g == 2 ? a.w[2] : (g == 1 ? a.w[1] : a.w[0]);
+  uint16_t* const y = g == 2 ? a.y[2] : (g == 1 ? a.y[1] : a.y[0]);
+  const int N = g == 2 ? a.N[2] : (g == 1 ? a.N[1] : a.N[0]);
+  const int tile0 = g == 2 ? a.tile0[2] : (g == 1 ? a.tile0[1] : 0);
+  const uint32_t* const t = g == 2 ? a.t[2] : (g == 1 ? a.t[1] : a.t[0]);
+  const uint32_t tn = g == 2 ? a.tn[2] : (g == 1 ? a.tn[1] : a.tn[0]);
+  const int m0 = mb * G::BM, n0 = (nb - tile0) * G::BN;
   const int c0 = (int)((int64_t)kpi * a.steps / a.kp);
   const int c1 = (int)((int64_t)(kpi + 1) * a.steps / a.kp);
   typename G::Ctx cx;
-  const int rows = min(G::BM, a.M - m0), cols = min(G::BN, a.N - n0);
-  G::setup(cx, a.K, a.tn, n0, cols);
+  const int rows = min(G::BM, a.M - m0), cols = min(G::BN, N - n0);
+  G::setup(cx, a.K, tn, n0, cols);
   // the buffers end with the tile's last row: reads past it return zeros
   cx.x = buffer_rsrc(a.x + (int64_t)m0 * a.K, (uint32_t)rows * cx.xstride);
-  cx.w = buffer_rsrc(a.w + (int64_t)n0 * (cx.wstride / 4), (uint32_t)cols * cx.wstride);
-  cx.t = buffer_rsrc(a.t, a.tn * (uint32_t)cx.groups * 4u);
+  cx.w = buffer_rsrc(w + (int64_t)n0 * (cx.wstride / 4), (uint32_t)cols * cx.wstride);
+  cx.t = buffer_rsrc(t, (tn * (uint32_t)(cx.groups - 1) + (uint32_t)N) * 4u);
   typename G::Acc acc;
 #pragma unroll
   for (int i = 0; i < MT; ++i)
@@ -658,8 +675,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qmm_gemm_kernel(GemmArgs a) {
     for (int p = threadIdx.x; p < G::BM * PPR; p += G::THREADS) {
       const int m = p / PPR, n = (p % PPR) * 8;
       const u32x4 v = *reinterpret_cast<const u32x4*>(dfmi_smem + m * G::YROW + n * 2);
-      if (m0 + m < a.M && n0 + n < a.N)
-        *reinterpret_cast<u32x4*>(a.y + (int64_t)(m0 + m) * a.N + n0 + n) = v;
+      if (m0 + m < a.M && n0 + n < N)
+        *reinterpret_cast<u32x4*>(y + (int64_t)(m0 + m) * N + n0 + n) = v;
     }
     return;
   }
@@ -670,7 +687,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qmm_gemm_kernel(GemmArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int m = m0 + row + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3), n = n0 + col + 32 * j;
-        if (m < a.M && n < a.N) a.y[(int64_t)m * a.N + n] = Num<Tag>::f2h(acc.v[i][j][r]);
+        if (m < a.M && n < N) y[(int64_t)m * N + n] = Num<Tag>::f2h(acc.v[i][j][r]);
       }
 }
 
@@ -680,18 +697,20 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qmm_gemm_kernel(GemmArgs a) {
 // kernel instead took 1.1 us per split on one CU: [77,5120] x [5120,5120] in 6
 // splits 20.6 us.)
 template <typename Tag, int MT, int NT, int WM, int WN>
-__global__ __launch_bounds__(256) void qmm_gemm_sum_kernel(const float* partials, uint16_t* y,
-                                                           int M, int N, int tiles_m, int kp,
-                                                           int vec) {
+__global__ __launch_bounds__(256) void qmm_gemm_sum_kernel(GemmArgs a) {
   constexpr int BM = 32 * MT * WM, BN = 32 * NT * WN, TILE = BM * BN, PER = TILE / 1024;
   const int tile = blockIdx.x / PER, e = ((blockIdx.x % PER) * 256 + threadIdx.x) * 4;
+  const int nb = tile / a.tiles_m, g = gemm_seg(a, nb), kp = a.kp;
+  uint16_t* const y = g == 2 ? a.y[2] : (g == 1 ? a.y[1] : a.y[0]);
+  const int N = g == 2 ? a.N[2] : (g == 1 ? a.N[1] : a.N[0]);
+  const int tile0 = g == 2 ? a.tile0[2] : (g == 1 ? a.tile0[1] : 0);
   // e: wavefront, row block and column tile, register, lane
   const int wave = e / (MT * NT * 1024), ij = e / 1024 % (MT * NT), r = e / 64 % 16, lane = e % 64;
-  const int m = (tile % tiles_m) * BM + (wave / WN) * 32 * MT + (ij / NT) * 32 + 8 * (r >> 2) +
+  const int m = (tile % a.tiles_m) * BM + (wave / WN) * 32 * MT + (ij / NT) * 32 + 8 * (r >> 2) +
                 4 * (lane >> 5) + (r & 3);
-  const int n = (tile / tiles_m) * BN + (wave % WN) * 32 * NT + (ij % NT) * 32 + (lane & 31);
-  if (m >= M || n >= N) return;
-  const float* p = partials + (int64_t)tile * kp * TILE + e;
+  const int n = (nb - tile0) * BN + (wave % WN) * 32 * NT + (ij % NT) * 32 + (lane & 31);
+  if (m >= a.M || n >= N) return;
+  const float* p = a.partials + (int64_t)tile * kp * TILE + e;
   f32x4 sum = zero4();
   for (int k0 = 0; k0 < kp; k0 += 4) {
     f32x4 t[4];
@@ -704,7 +723,7 @@ __global__ __launch_bounds__(256) void qmm_gemm_sum_kernel(const float* partials
       for (int c = 0; c < 4; ++c) sum[c] += k0 + k < kp ? t[k][c] : 0.f;
   }
   uint16_t* out = y + (int64_t)m * N + n;
-  if (vec) {
+  if (a.vec) {
     u32x2 v;
     v.x = (uint32_t)Num<Tag>::f2h(sum.x) | ((uint32_t)Num<Tag>::f2h(sum.y) << 16);
     v.y = (uint32_t)Num<Tag>::f2h(sum.z) | ((uint32_t)Num<Tag>::f2h(sum.w) << 16);
@@ -730,8 +749,7 @@ static void gemm_launch_cfg(const GemmArgs& a, hipStream_t st) {
                      dim3(a.tiles_m * a.tiles_n * a.kp), dim3(G::THREADS), G::LDS_BYTES, st, a);
   if (a.kp > 1)
     hipLaunchKernelGGL((qmm_gemm_sum_kernel<Tag, MT, NT, WM, WN>),
-                       dim3(a.tiles_m * a.tiles_n * (G::BM * G::BN / 1024)), dim3(256), 0, st,
-                       a.partials, a.y, a.M, a.N, a.tiles_m, a.kp, a.vec);
+                       dim3(a.tiles_m * a.tiles_n * (G::BM * G::BN / 1024)), dim3(256), 0, st, a);
 }
 
 // cfg: index into kGemmCfgs (dfmi_gemm.hip)

@@ -33,13 +33,16 @@ struct GemmPlan {
 // eight K x N from 1024 x 512 to 17408 x 5120, MI355X, gs 64, 4-bit, bf16):
 // what the rule picks is 1.2 % slower in the mean than the best of them all,
 // 14 % at worst; 64 x 128, 32 x 256 and 128 x 256 tiles would add 0.9 %.
-static GemmPlan gemm_plan(int64_t M, int64_t K, int64_t N, size_t max_partials) {
+static GemmPlan gemm_plan(int64_t M, int64_t K, const int64_t* Ns, int nseg,
+                          size_t max_partials) {
   const int steps = (int)((K + kGemmK - 1) / kGemmK);
   GemmPlan best{};
   double best_t = 0;
   for (int c = 0; c < kNumGemmCfgs; ++c) {
     const GemmCfg& g = kGemmCfgs[c];
-    const int64_t tm = (M + g.bm - 1) / g.bm, tn = (N + g.bn - 1) / g.bn, tiles = tm * tn;
+    int64_t tm = (M + g.bm - 1) / g.bm, tn = 0;
+    for (int i = 0; i < nseg; ++i) tn += (Ns[i] + g.bn - 1) / g.bn;
+    const int64_t tiles = tm * tn;
     for (int kp = 1; kp <= 16 && 2 * kp <= std::max(steps, 2); ++kp) {
       const size_t bytes = kp > 1 ? (size_t)tiles * kp * g.bm * g.bn * 4u : 0;
       if (bytes > max_partials) break;
@@ -73,50 +76,92 @@ bool gemm_shape(int64_t M, int64_t K, int64_t N, int gs) {
 }
 
 size_t gemm_workspace_bytes(int64_t M, int64_t K, int64_t N, int gs) {
-  return kGemmWsOffset + table_bytes(K, N, gs) + gemm_plan(M, K, N, kGemmMaxPartials).partials;
+  return kGemmWsOffset + table_bytes(K, N, gs) +
+         gemm_plan(M, K, &N, 1, kGemmMaxPartials).partials;
 }
 
-int gemm_launch(const void* x, int x_dtype, const uint32_t* w, const void* scales,
-                const void* biases, const uint32_t* pairs, int64_t pair_stride, void* y,
-                int64_t M, int64_t K, int64_t N, int gs, int bits, void* workspace,
-                size_t workspace_bytes, hipStream_t st) {
-  char* ws = static_cast<char*>(workspace);
-  size_t left = ws && workspace_bytes > kGemmWsOffset && aligned16(ws)
-                    ? workspace_bytes - kGemmWsOffset : 0;
-  ws += kGemmWsOffset;
-  if (!pairs) {
-    // the table into the workspace, for this call
-    const size_t need = table_bytes(K, N, gs);
-    if (left < need) return kGemmNotTaken;
-    uint32_t* t = reinterpret_cast<uint32_t*>(ws);
-    const int rc = dfmi_sb_pairs(scales, biases, x_dtype, N, K / gs, t, st);
-    if (rc != DFMI_OK) return rc;
-    pairs = t;
-    pair_stride = N;
-    ws += need;
-    left -= need;
+size_t gemm_multi_workspace_bytes(int64_t M, int64_t K, const int64_t* Ns, int nseg, int gs) {
+  size_t tables = 0;
+  for (int i = 0; i < nseg; ++i) tables += table_bytes(K, Ns[i], gs);
+  return kGemmWsOffset + tables + gemm_plan(M, K, Ns, nseg, kGemmMaxPartials).partials;
+}
+
+// the planned launch of a whose matrices, table and rows are set
+static int gemm_run(GemmArgs& a, int x_dtype, int gs, int bits, char* ws, size_t left,
+                    hipStream_t st) {
+  int64_t Ns[kGemmMaxSeg];
+  bool vec = true;
+  for (int i = 0; i < a.nseg; ++i) {
+    Ns[i] = a.N[i];
+    vec = vec && aligned16(a.y[i]) && a.N[i] % 8 == 0;
   }
-  const GemmPlan p = gemm_plan(M, K, N, std::min(left, kGemmMaxPartials));
-  GemmArgs a{};
-  a.x = static_cast<const uint16_t*>(x);
-  a.w = w;
-  a.t = pairs;
-  a.y = static_cast<uint16_t*>(y);
+  const GemmPlan p = gemm_plan(a.M, a.K, Ns, a.nseg, std::min(left, kGemmMaxPartials));
+  const int bn = kGemmCfgs[p.cfg].bn;
+  int tile = 0;
+  for (int i = 0; i < a.nseg; ++i) {
+    a.tile0[i] = tile;
+    tile += (a.N[i] + bn - 1) / bn;
+  }
   a.partials = reinterpret_cast<float*>(ws);
-  a.M = (int)M;
-  a.K = (int)K;
-  a.N = (int)N;
-  a.tn = (uint32_t)(pair_stride ? pair_stride : N);
-  a.steps = (int)((K + kGemmK - 1) / kGemmK);
+  a.steps = (a.K + kGemmK - 1) / kGemmK;
   a.tiles_m = p.tiles_m;
   a.tiles_n = p.tiles_n;
   a.kp = p.kp;
-  a.vec = aligned16(y) && N % 8 == 0;
+  a.vec = vec;
   if (x_dtype == DFMI_BF16)
     bits == 4 ? gemm_launch_bf16_4(p.cfg, gs, a, st) : gemm_launch_bf16_8(p.cfg, gs, a, st);
   else
     bits == 4 ? gemm_launch_f16_4(p.cfg, gs, a, st) : gemm_launch_f16_8(p.cfg, gs, a, st);
   return check_launch("dfmi_qmm_affine (gemm)");
+}
+
+// what of a caller's workspace is free for the tables and partial tiles
+static size_t gemm_space(void* workspace, size_t bytes, char*& ws) {
+  ws = static_cast<char*>(workspace) + kGemmWsOffset;
+  return workspace && aligned16(workspace) && bytes > kGemmWsOffset ? bytes - kGemmWsOffset : 0;
+}
+
+int gemm_launch(const void* x, int x_dtype, const dfmi_qmm_segment* segs, int nseg,
+                const uint32_t* fused, int64_t pair_stride, int64_t M, int64_t K, int gs,
+                int bits, void* workspace, size_t workspace_bytes, hipStream_t st) {
+  char* ws;
+  size_t left = gemm_space(workspace, workspace_bytes, ws);
+  // matrices without a table: theirs into the workspace, for this call
+  size_t need = 0;
+  int64_t cols = 0;
+  for (int i = 0; i < nseg; ++i) {
+    if (!fused && !segs[i].sb_pairs) need += table_bytes(K, segs[i].N, gs);
+    cols += segs[i].N;
+  }
+  if (left < need) return kGemmNotTaken;
+  GemmArgs a{};
+  a.x = static_cast<const uint16_t*>(x);
+  a.nseg = nseg;
+  a.M = (int)M;
+  a.K = (int)K;
+  for (int i = 0; i < nseg; ++i) {
+    const int64_t N = segs[i].N;
+    a.w[i] = segs[i].w_q;
+    a.y[i] = static_cast<uint16_t*>(segs[i].y);
+    a.N[i] = (int)N;
+    if (fused) {
+      a.t[i] = fused;
+      a.tn[i] = (uint32_t)cols;
+      fused += N;
+    } else if (segs[i].sb_pairs) {
+      a.t[i] = segs[i].sb_pairs;
+      a.tn[i] = (uint32_t)(pair_stride ? pair_stride : N);
+    } else {
+      uint32_t* t = reinterpret_cast<uint32_t*>(ws);
+      const int rc = dfmi_sb_pairs(segs[i].scales, segs[i].biases, x_dtype, N, K / gs, t, st);
+      if (rc != DFMI_OK) return rc;
+      a.t[i] = t;
+      a.tn[i] = (uint32_t)N;
+      ws += table_bytes(K, N, gs);
+      left -= table_bytes(K, N, gs);
+    }
+  }
+  return gemm_run(a, x_dtype, gs, bits, ws, left, st);
 }
 
 }  // namespace dfmi

@@ -42,10 +42,13 @@ inline bool stream_eligible(int64_t M, int64_t K, int64_t N, int gs, int bits = 
 constexpr int kGemmNotTaken = 1;
 bool gemm_shape(int64_t M, int64_t K, int64_t N, int gs);
 size_t gemm_workspace_bytes(int64_t M, int64_t K, int64_t N, int gs);
-int gemm_launch(const void* x, int x_dtype, const uint32_t* w, const void* scales,
-                const void* biases, const uint32_t* pairs, int64_t pair_stride, void* y,
-                int64_t M, int64_t K, int64_t N, int gs, int bits, void* workspace,
-                size_t workspace_bytes, hipStream_t st);
+size_t gemm_multi_workspace_bytes(int64_t M, int64_t K, const int64_t* Ns, int nseg, int gs);
+// fused: the matrices' tables side by side, or null (their own sb_pairs, rows
+// pair_stride apart if not 0).  More than one matrix: every N >= 1 and a
+// multiple of 4.
+int gemm_launch(const void* x, int x_dtype, const dfmi_qmm_segment* segs, int nseg,
+                const uint32_t* fused, int64_t pair_stride, int64_t M, int64_t K, int gs,
+                int bits, void* workspace, size_t workspace_bytes, hipStream_t st);
 
 }  // namespace dfmi
 

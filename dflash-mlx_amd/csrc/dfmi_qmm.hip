@@ -953,6 +953,20 @@ static int launch_streaming(const void* x, int x_dtype, const StreamSegs& segs, 
   return run_streaming(L, x, st);
 }
 
+// One matrix-core launch of two or three matrices: each takes that kernel and
+// starts on a 16-byte boundary of a table of them all.  (A layer's q/k/v, o,
+// gate/up and down over 77 rows of 5120, 17408 wide: 144 us, with a launch for
+// each matrix 163: fewer nearly empty last waves and split sums.)
+static bool use_gemm_multi(int64_t M, int64_t K, const int64_t* Ns, int nseg, int gs) {
+  if (nseg < 2 || nseg > 3) return false;
+  int64_t sum = 0;
+  for (int i = 0; i < nseg; ++i) {
+    if (Ns[i] < 1 || Ns[i] % 4) return false;
+    sum += Ns[i];
+  }
+  return gemm_shape(M, K, sum, gs);
+}
+
 // Shared-activation launches take the streaming kernel when every matrix
 // does (their blocks then form one grid); the columns of that grid, 64 per
 // block, or 0.
@@ -1068,8 +1082,9 @@ static int qmm_affine(const void* x, int x_dtype, const uint32_t* w_q, const voi
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (use_gemm(M, K, N, group_size, tuning)) {
-    rc = gemm_launch(x, x_dtype, w_q, scales, biases, sb_pairs, sb_stride, y, M, K, N, group_size,
-                     bits, workspace, workspace_bytes, st);
+    const dfmi_qmm_segment seg{w_q, scales, biases, y, N, sb_pairs};
+    rc = gemm_launch(x, x_dtype, &seg, 1, nullptr, sb_stride, M, K, group_size, bits, workspace,
+                     workspace_bytes, st);
     if (rc != kGemmNotTaken) return rc;
   }
   // 8-bit: the streaming kernel where it applies, else the register-load kernel
@@ -1255,6 +1270,8 @@ extern "C" size_t dfmi_qmm_multi_workspace_bytes(int64_t M, int64_t K, const int
   size_t ws = 0;
   for (int i = 0; i < nseg; ++i)
     ws = std::max(ws, dfmi_qmm_workspace_bytes_ex(M, K, Ns[i], group_size, bits, nullptr));
+  if (use_gemm_multi(M, K, Ns, nseg, group_size))
+    ws = std::max(ws, gemm_multi_workspace_bytes(M, K, Ns, nseg, group_size));
   return ws;
 }
 
@@ -1314,6 +1331,11 @@ static int qmm_multi(const void* x, int x_dtype, const dfmi_qmm_segment* segs, i
     m.fused = fused;
     return launch_streaming(x, x_dtype, m, M, K, cols, group_size, bits, nullptr, workspace,
                             workspace_bytes, static_cast<hipStream_t>(stream));
+  }
+  if (use_gemm_multi(M, K, Ns, nseg, group_size)) {
+    const int rc = gemm_launch(x, x_dtype, segs, nseg, fused, 0, M, K, group_size, bits,
+                               workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+    if (rc != kGemmNotTaken) return rc;
   }
   // one launch per matrix, in order on the stream (they may share the workspace)
   for (int i = 0; i < nseg; ++i) {

@@ -31,6 +31,7 @@ from .verify_qmm import (
     _m4_ksplit_np_shape,
     _resolve_m16_ktmpl_variant,
     current_stream,
+    qmm_fused_launch,
     qmm_launch,
     quantized_matmul,
     verify_matmul,
@@ -218,7 +219,10 @@ class _VerifyState:
         if self.pairs is None and torch.cuda.is_current_stream_capturing():
             return None
         t = self.pair_table()
-        return t if self.vers == (self.s._version, self.b._version) else None
+        return t if self.table_current() else None
+
+    def table_current(self) -> bool:
+        return self.vers is not None and self.vers == _runtime.versions((self.s, self.b))
 
     def pair_table(self):
         """The pair table (built on first use; None while a graph is being
@@ -230,7 +234,7 @@ class _VerifyState:
                 _warn_capture_without_table()
                 return None
             self.pairs = _runtime.build_sb_pairs(self.s, self.b)
-            self.vers = (self.s._version, self.b._version)
+            self.vers = _runtime.versions((self.s, self.b))
         return self.pairs
 
     def record(self, m: int, st: int, x: torch.Tensor) -> LaunchRecord:
@@ -315,10 +319,15 @@ def _build_dispatch(obj: VerifyQuantizedLinear, *, enable_qmm: Optional[bool] = 
                 y = y.view(*shp[:-1], N)
             elif (x.dtype == sdt and x.is_cuda and m > 32 and kx == K and mode == "affine"
                   and (t := state.current_table(obj)) is not None):
-                # many rows: the stock route, with the table the module holds
-                y = qmm_launch(_runtime.aligned_contiguous(x.reshape(m, kx)), state.w, state.s,
-                               state.b, N, gs, bits, pairs=t,
-                               pair_stride=state.stride).view(*shp[:-1], N)
+                # many rows: the stock route, with the table the module holds,
+                # or as one launch with its siblings
+                grp = state.group
+                y = (grp.product(state.gidx, x, m, current_stream(x.get_device()))
+                     if grp is not None and not x.is_inference() else None)
+                if y is None:
+                    y = qmm_launch(_runtime.aligned_contiguous(x.reshape(m, kx)), state.w, state.s,
+                                   state.b, N, gs, bits, pairs=t, pair_stride=state.stride)
+                y = y.view(*shp[:-1], N)
             else:
                 y = _stock(x)
             return y + bias if bias is not None else y
@@ -395,10 +404,11 @@ _SIBLING_SETS = (("q_proj", "k_proj", "v_proj"), ("gate_proj", "up_proj"))
 class SiblingGroup:
     """Verify modules of one parent that read the same input (q/k/v, gate/up).
 
-    The first member called with an input of at most 32 rows computes the
-    product of every active member in one shared-activation launch
-    (``dfmi_qmm_run`` on the group's prepared launch, the members' pair
-    tables side by side in one combined table); each other member returns
+    The first member called with an input computes the product of every
+    active member in one shared-activation launch (``dfmi_qmm_run`` on the
+    group's prepared launch, the members' pair tables side by side in one
+    combined table; beyond 32 rows ``dfmi_qmm_affine_multi_fused`` where every
+    member is active and has such a table); each other member returns
     its own product when it is called with the same tensor object, unchanged
     (same ``_version``) and on the same stream -- in the model's call order,
     with no change to the model code.  The group holds that input until every
@@ -421,29 +431,28 @@ class SiblingGroup:
         self.stride = stride
         self._miss = [0] * len(self.states)
         self._recs: dict = {}
-        self._x = None
-        self._ver = -1
-        self._st = 0
-        self._ys: dict = {}
+        # (input, its version, where it ran, outputs not yet taken, the
+        # weights' versions), replaced as one: several threads may call
+        self._pending: Optional[tuple] = None
 
     def reset(self) -> None:
         """Forget any pending outputs (and the held input) and the miss
         counts, and take every member back into the shared launch."""
-        self._x, self._ver, self._st, self._ys = None, -1, 0, {}
+        self._pending = None
         self._miss = [0] * len(self.states)
         self.active = tuple(range(len(self.states)))
 
-    def _record(self, m: int, st: int, x: torch.Tensor) -> LaunchRecord:
-        key = (m, st, x.dtype, self.active)
+    def _record(self, m: int, st: int, x: torch.Tensor, active) -> LaunchRecord:
+        key = (m, st, x.dtype, active)
         rec = self._recs.get(key)
         if rec is None:
-            sts = [self.states[j] for j in self.active]
+            sts = [self.states[j] for j in active]
             first = sts[0]
             tabs = [st_.pair_table() for st_ in sts]
             # the combined table serves the launch of every member (the
             # fused kernel: two or three matrices of fewer than 2^16 rows);
             # otherwise each matrix reads its column slice of it
-            if (self.fused is not None and len(self.active) == len(self.states)
+            if (self.fused is not None and len(active) == len(self.states)
                     and 2 <= len(sts) <= 3 and all(q.N < 65536 for q in sts)):
                 rec = LaunchRecord(m, first.K, x.dtype, x.device,
                                    [(q.w, q.s, q.b) for q in sts], first.gs, first.bits,
@@ -472,48 +481,68 @@ class SiblingGroup:
                                 torch.cuda.current_device())
             for m in (16, 4):
                 x = torch.zeros((m, first.K), dtype=dtype, device=dev)
-                rec = self._record(m, st, x)
+                rec = self._record(m, st, x, self.active)
                 rec.run(x, [torch.empty((m, self.states[j].N), dtype=dtype, device=dev)
                              for j in self.active], st)
         self.reset()
 
+    def _takes_many(self, active) -> bool:
+        """More than 32 rows run as one launch: every member active, their
+        tables side by side and built from the scales as they are."""
+        return (self.fused is not None and 2 <= len(self.states) <= 3
+                and len(active) == len(self.states)
+                and all(q.table_current() and not q.w.is_inference() for q in self.states))
+
     def product(self, idx: int, x: torch.Tensor, m: int, st: int) -> Optional[torch.Tensor]:
         """Member idx's [m, N] product of x, or None when idx is not in the
         shared launch (the member then launches alone)."""
-        ys = self._ys
-        if ys and self._x is x and self._ver == x._version and self._st == st:
-            y = ys.pop(idx, None)
+        many = m > 32
+        # (a captured launch computes nothing until its graph is replayed)
+        where = (st, torch.cuda.is_current_stream_capturing()) if many else st
+        pending = self._pending
+        if pending is not None and pending[0] is x and pending[1] == x._version \
+                and pending[2] == where:
+            y = pending[3].pop(idx, None)
             if y is not None:
                 self._miss[idx] = 0
-                if not ys:
-                    self._x = None  # every output taken: let the input go
-                return y
-        if idx not in self.active:
+                if not pending[3] and self._pending is pending:
+                    self._pending = None  # every output taken: let the input go
+                if pending[4] is None or pending[4][idx] == self.states[idx].w._version:
+                    return y
+        active = self.active
+        if idx not in active:
             return None
-        if ys:  # members that did not take the previous launch's output
+        if many and not self._takes_many(active):
+            return None
+        if pending is not None and pending[3]:  # members that did not take their output
             keep = []
-            for j in self.active:
-                if j in ys:
+            for j in active:
+                if j in pending[3]:
                     self._miss[j] += 1
                 if self._miss[j] < 2:
                     keep.append(j)
-            self.active = tuple(keep) if len(keep) >= 2 else ()
-            self._ys = {}
-            if idx not in self.active:
-                self._x = None
+            self.active = active = tuple(keep) if len(keep) >= 2 else ()
+            self._pending = None
+            if idx not in active or (many and not self._takes_many(active)):
                 return None
         x2 = x.reshape(m, int(x.shape[-1]))
         if not x2.is_contiguous() or x2.data_ptr() & 15:
             x2 = _runtime.aligned_contiguous(x2)
-        rec = self._recs.get((m, st, x.dtype, self.active)) or self._record(m, st, x)
         outs = [torch.empty((m, self.states[j].N), dtype=x.dtype, device=x.device)
-                for j in self.active]
-        rec.run(x2, outs, st)
-        ys = dict(zip(self.active, outs))
+                for j in active]
+        vers = None
+        if many:
+            first = self.states[0]
+            vers = [q.w._version for q in self.states]
+            qmm_fused_launch(x2, [(q.w, q.s, q.b) for q in self.states], self.fused, first.gs,
+                             first.bits, outs)
+        else:
+            rec = self._recs.get((m, st, x.dtype, active)) or self._record(m, st, x, active)
+            rec.run(x2, outs, st)
+        ys = dict(zip(active, outs))
         y = ys.pop(idx)
         self._miss[idx] = 0
-        self._ys = ys
-        self._x, self._ver, self._st = (x, x._version, st) if ys else (None, -1, 0)
+        self._pending = (x, x._version, where, ys, vers) if ys else None
         return y
 
 

@@ -190,6 +190,7 @@ def qmm_multi_launch(x2: torch.Tensor, mats, group_size: int, bits: int,
     ws, ws_bytes = space(dev, need) if need else (0, 0)
     # two or three matrices with tables: the tables side by side, so that the
     # fused kernel starts its first loads without reading a segment table
+    # (many rows: the matrix-core kernel takes them apart as well)
     fused = (_runtime.FUSED_PAIRS.get(tables)
              if 2 <= n <= 3 and not _runtime.many_rows(M) and all(t is not None for t in tables) else None)
     if fused is not None:
@@ -203,6 +204,30 @@ def qmm_multi_launch(x2: torch.Tensor, mats, group_size: int, bits: int,
                                        _runtime.stream_ptr(dev))
     _lib.check(status, "dfmi_qmm_affine_multi")
     return ys
+
+
+def qmm_fused_launch(x2: torch.Tensor, mats, fused: torch.Tensor, group_size: int, bits: int,
+                     outs) -> None:
+    """One ``dfmi_qmm_affine_multi_fused`` launch of the sibling matrices
+    ``mats = [(w, scales, biases), ...]`` (2 or 3) whose pair tables stand side
+    by side in ``fused``, into ``outs``."""
+    lib = _lib.load()
+    M, K = int(x2.shape[0]), int(x2.shape[1])
+    dev = x2.device
+    n = len(mats)
+    segs = (_lib.QmmSegment * n)()
+    ns = (ctypes.c_int64 * n)()
+    for i, ((w, sc, bi), y) in enumerate(zip(mats, outs)):
+        segs[i].w_q, segs[i].scales, segs[i].biases = w.data_ptr(), sc.data_ptr(), bi.data_ptr()
+        segs[i].y, segs[i].N = y.data_ptr(), int(w.shape[0])
+        ns[i] = int(w.shape[0])
+    need = int(lib.dfmi_qmm_multi_workspace_bytes(M, K, ns, n, int(group_size), int(bits)))
+    space = _runtime.optional_workspace if _runtime.many_rows(M) else _runtime.workspace
+    ws, ws_bytes = space(dev, need) if need else (0, 0)
+    status = lib.dfmi_qmm_affine_multi_fused(
+        x2.data_ptr(), _runtime.dtype_code(x2.dtype), segs, n, fused.data_ptr(), M, K,
+        int(group_size), int(bits), ws, ws_bytes, _runtime.stream_ptr(dev))
+    _lib.check(status, "dfmi_qmm_affine_multi_fused")
 
 
 _raw_stream = torch._C._cuda_getCurrentRawStream

@@ -232,11 +232,12 @@ size_t dfmi_qmm_noalloc_scratch_bytes(void);
  * an MLP (dflash_mlx/verify_linear.py:266-286, one call per
  * VerifyQuantizedLinear) -- so that the layer pays one launch, one pipeline
  * fill and one grid for them: the row blocks of all W_i form one streaming
- * grid.  Shapes outside the streaming kernel (M > 32, K % 256 != 0, ...) run
- * as nseg dfmi_qmm_affine calls on the stream, in order.  Each y_i is within
- * fp32 summation order of what dfmi_qmm_affine returns for W_i alone (the two
- * may split K differently); the result does not depend on scheduling.  The
- * workspace is dfmi_qmm_multi_workspace_bytes bytes, zero-filled when
+ * grid.  At M > 32 two or three matrices (each N a multiple of 4) form one
+ * matrix-core grid likewise, given the workspace or their pair tables.  Other
+ * shapes (K % 256 != 0, ...) run as nseg dfmi_qmm_affine calls on the stream,
+ * in order.  Each y_i is within fp32 summation order of what dfmi_qmm_affine
+ * returns for W_i alone (the two may split K differently); the result does not
+ * depend on scheduling.  The workspace is dfmi_qmm_multi_workspace_bytes bytes, zero-filled when
  * created.
  */
 typedef struct dfmi_qmm_segment {

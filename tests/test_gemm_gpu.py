@@ -118,27 +118,129 @@ def test_rows_with_infinities_stay_apart(dev):
     assert not torch.isfinite(got[[11, 40, 69]]).any()
 
 
-def test_module_many_rows(dev):
-    """A verify module's many-row call equals the stock operator bit for bit,
-    alone and as a sibling, also after its scales change in place."""
+@pytest.mark.parametrize("M,K,Ns,gs,bits,dtype", [
+    (33, 64, (4, 260), 32, 4, "bf16"), (77, 1152, (132, 4, 388), 64, 4, "f16"),
+    (200, 640, (512, 128), 128, 8, "bf16"), (65, 4096, (256, 260, 64), 64, 4, "bf16"),
+])
+def test_matrices_in_one_launch(dev, M, K, Ns, gs, bits, dtype):
+    """Two and three matrices, their tables side by side, in one launch: each
+    within the bound, with partial column tiles at the seams, also without a
+    workspace (no K split); the launch beside it, one per matrix, too."""
+    import torch
+
+    from dflash_mlx_amd import _lib, _runtime, verify_qmm as vq
+
+    cases, mats, x = [], [], None
+    for i, N in enumerate(Ns):
+        case, (xi, w, s, b) = _case(dev, M, K, N, gs, bits, dtype, seed=40 + i)
+        x, cx = (xi, case[0]) if x is None else (x, cx)
+        cases.append((cx,) + case[1:])
+        mats.append((w, s, b))
+
+    def check(ys):
+        for y, case in zip(ys, cases):
+            _check(from_dev(y, dtype), case, gs, bits, dtype)
+
+    one = vq.quantized_matmul_multi(x, mats, group_size=gs, bits=bits)
+    check(one)
+    check([vq.quantized_matmul(x, *m, group_size=gs, bits=bits) for m in mats])
+    fused = torch.cat([_runtime.build_sb_pairs(s, b) for _, s, b in mats], dim=1).contiguous()
+    outs = [torch.full_like(y, float("nan")) for y in one]
+    vq.qmm_fused_launch(x, mats, fused, gs, bits, outs)
+    assert all(torch.equal(a, b) for a, b in zip(one, outs))
+    segs = (_lib.QmmSegment * len(mats))()
+    for g, (w, s, b), y in zip(segs, mats, outs):
+        g.w_q, g.scales, g.biases = w.data_ptr(), s.data_ptr(), b.data_ptr()
+        g.y, g.N = y.fill_(float("nan")).data_ptr(), int(w.shape[0])
+    rc = _lib.load().dfmi_qmm_affine_multi_fused(
+        x.data_ptr(), _runtime.dtype_code(x.dtype), segs, len(mats), fused.data_ptr(), M, K, gs,
+        bits, None, 0, _runtime.stream_ptr(x.device))
+    assert rc == _lib.DFMI_OK
+    check(outs)
+
+
+def test_many_rows_in_inference_mode(dev):
+    """Tensors that count no versions (made under inference mode) are taken,
+    by the operators and by modules, and weights changed in place between two
+    siblings' calls are seen."""
     import torch
     from torch import nn
 
     from dflash_mlx_amd import verify_linear as vl, verify_qmm as vq
 
-    K, gs, M = 512, 64, 45
+    M, K, N, gs = 45, 512, 256, 64
+    case, (x, w, s, b) = _case(dev, M, K, N, gs, 4, "bf16", seed=31)
+    with torch.inference_mode():
+        xi, wi, si, bi = (t.clone() for t in (x, w, s, b))
+        _check(from_dev(vq.quantized_matmul(xi, wi, si, bi, group_size=gs, bits=4), "bf16"),
+               case, gs, 4, "bf16")
+        for y in vq.quantized_matmul_multi(xi, [(w, s, b), (wi, si, bi)], group_size=gs, bits=4):
+            _check(from_dev(y, "bf16"), case, gs, 4, "bf16")
     root = nn.Module()
     root.mlp = nn.Module()
-    x = None
-    for i, (name, N) in enumerate((("gate_proj", 384), ("up_proj", 640), ("down_proj", 256))):
-        _, (xi, w, s, b) = _case(dev, M, K, N, gs, 4, "bf16", seed=20 + i)
-        x = xi if x is None else x
-        setattr(root.mlp, name, vl.QuantizedLinear(w, s, b, group_size=gs, bits=4))
+    for name in ("gate_proj", "up_proj"):
+        setattr(root.mlp, name, vl.QuantizedLinear(w.clone(), s.clone(), b.clone(),
+                                                   group_size=gs, bits=4))
     vl.install_verify_linears(root, enable_qmm=True)
-    for change in (False, True):
-        for name in ("gate_proj", "up_proj", "down_proj"):
-            m = getattr(root.mlp, name)
-            if change:
-                m.scales.mul_(1.5)
-            want = vq.quantized_matmul(x, m.weight, m.scales, m.biases, group_size=gs, bits=4)
-            assert torch.equal(m(x), want), name
+    gate, up = root.mlp.gate_proj, root.mlp.up_proj
+    with torch.inference_mode():
+        for m in (gate, up):
+            _check(from_dev(m(x.clone()), "bf16"), case, gs, 4, "bf16")
+    gate(x)
+    up.weight.zero_()
+    want = vq.quantized_matmul(x, up.weight, up.scales, up.biases, group_size=gs, bits=4)
+    assert torch.equal(up(x), vq.quantized_matmul_multi(
+        x, [(m.weight, m.scales, m.biases) for m in (gate, up)], group_size=gs, bits=4)[1])
+    assert torch.allclose(up(x).float(), want.float(), rtol=2 ** -7, atol=0)
+
+
+def test_module_many_rows(dev):
+    """A verify module's many-row call: alone it equals the stock operator bit
+    for bit, siblings the shared launch of quantized_matmul_multi (each within
+    the bound), also with rows split over workgroups, in any call order, under
+    graph replay, and after scales change in place (then the stock route)."""
+    import torch
+    from torch import nn
+
+    from dflash_mlx_amd import verify_linear as vl, verify_qmm as vq
+
+    K, gs = 2048, 64
+    names = (("gate_proj", 384), ("up_proj", 644), ("down_proj", 256))
+    for M in (45, 200):
+        root, cases, x = nn.Module(), {}, None
+        root.mlp = nn.Module()
+        for i, (name, N) in enumerate(names):
+            case, (xi, w, s, b) = _case(dev, M, K, N, gs, 4, "bf16", seed=20 + i)
+            x, cx = (xi, case[0]) if x is None else (x, cx)
+            cases[name] = (cx,) + case[1:]
+            setattr(root.mlp, name, vl.QuantizedLinear(w, s, b, group_size=gs, bits=4))
+        vl.install_verify_linears(root, enable_qmm=True)
+        gate, up, down = (getattr(root.mlp, n) for n, _ in names)
+        want = vq.quantized_matmul_multi(
+            x, [(m.weight, m.scales, m.biases) for m in (gate, up)], group_size=gs, bits=4)
+        for first, second in ((0, 1), (1, 0)):
+            mods = (gate, up)
+            got = {first: mods[first](x), second: mods[second](x)}
+            assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+        for m, name in ((gate, "gate_proj"), (up, "up_proj")):
+            _check(from_dev(m(x), "bf16"), cases[name], gs, 4, "bf16")
+        stock = vq.quantized_matmul(x, down.weight, down.scales, down.biases, group_size=gs,
+                                    bits=4)
+        assert torch.equal(down(x), stock)
+        stream = torch.cuda.Stream()
+        stream.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(stream):
+            gate(x), up(x)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            g, u = gate(x), up(x)
+        for _ in range(3):
+            g.zero_(), u.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(g, want[0]) and torch.equal(u, want[1])
+        gate.scales.mul_(1.5)
+        for m in (gate, up, down):
+            want1 = vq.quantized_matmul(x, m.weight, m.scales, m.biases, group_size=gs, bits=4)
+            assert torch.equal(m(x), want1)
