@@ -31,9 +31,9 @@ def _mask_u8(mask: Optional[torch.Tensor], B: int, T: int) -> Optional[torch.Ten
 
 
 def _gate(g: torch.Tensor, B: int, T: int, Hv: int, Dk: int) -> Tuple[torch.Tensor, int]:
-    if g.dim() == 3 and tuple(g.shape) == (B, T, Hv):
+    if g.shape == (B, T, Hv):
         return g.contiguous(), 0
-    if g.dim() == 4 and tuple(g.shape) == (B, T, Hv, Dk):
+    if g.shape == (B, T, Hv, Dk):
         return g.contiguous(), 1
     raise ValueError(f"Unsupported gating shape {tuple(g.shape)}")
 
@@ -47,13 +47,13 @@ def gated_delta_kernel_with_tape(q: torch.Tensor, k: torch.Tensor, v: torch.Tens
     g [B,T,Hv] or [B,T,Hv,Dk], beta [B,T,Hv], state [B,Hv,Dv,Dk]."""
     for t, name in ((q, "q"), (k, "k"), (v, "v"), (g, "g"), (beta, "beta"), (state, "state")):
         _runtime.require_device(t, name)
-    B, T, Hk, Dk = (int(d) for d in k.shape)
-    Hv, Dv = int(v.shape[2]), int(v.shape[3])
+    B, T, Hk, Dk = k.shape
+    Hv, Dv = v.shape[2], v.shape[3]
     if Hv % Hk != 0:
         raise ValueError(f"Cannot align K heads {Hk} to V heads {Hv}")
-    if tuple(q.shape) != (B, T, Hk, Dk) or tuple(v.shape[:2]) != (B, T):
+    if q.shape != k.shape or v.shape[:2] != (B, T):
         raise ValueError("q, k [B,T,Hk,Dk] and v [B,T,Hv,Dv] must agree")
-    if tuple(beta.shape) != (B, T, Hv) or tuple(state.shape) != (B, Hv, Dv, Dk):
+    if beta.shape != (B, T, Hv) or state.shape != (B, Hv, Dv, Dk):
         raise ValueError("beta must be [B,T,Hv] and state [B,Hv,Dv,Dk]")
     if k.dtype != q.dtype or v.dtype != q.dtype:
         raise ValueError("q, k and v must share a dtype")
@@ -81,11 +81,11 @@ def tape_replay_kernel(tape: torch.Tensor, k: torch.Tensor, g: torch.Tensor,
     (fp32) with keys k [B,T,Hk,Dk] and gates g from ``state``."""
     for t, name in ((tape, "tape"), (k, "k"), (g, "g"), (state, "state")):
         _runtime.require_device(t, name)
-    B, T, Hk, Dk = (int(d) for d in k.shape)
-    Hv, Dv = int(tape.shape[2]), int(tape.shape[3])
+    B, T, Hk, Dk = k.shape
+    Hv, Dv = tape.shape[2], tape.shape[3]
     if Hv % Hk != 0:
         raise ValueError(f"Cannot align K heads {Hk} to tape heads {Hv}")
-    if tuple(tape.shape[:2]) != (B, T) or tuple(state.shape) != (B, Hv, Dv, Dk):
+    if tape.shape[:2] != (B, T) or state.shape != (B, Hv, Dv, Dk):
         raise ValueError("tape [B,T,Hv,Dv], k [B,T,Hk,Dk] and state [B,Hv,Dv,Dk] must agree")
     gc, per_key = _gate(g, B, T, Hv, Dk)
     m = _mask_u8(mask, B, T)

@@ -137,7 +137,7 @@ def qmm_launch(x2: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: 
     ``pair_stride`` columns; when None, the one cached for ``scales`` is used
     (built on first use).  The result does not depend on it."""
     lib = _lib.load()
-    M, K = int(x2.shape[0]), int(x2.shape[1])
+    M, K = x2.shape
     dev = x2.device
     y = out if out is not None else torch.empty((M, N), dtype=x2.dtype, device=dev)
     tptr = ctypes.byref(tuning) if tuning is not None else None
@@ -310,9 +310,13 @@ def _prepare(x, w, scales, biases):
     if scales.dtype != x.dtype or biases is None or biases.dtype != x.dtype:
         raise _lib.DfmiUnsupported(
             _lib.DFMI_EINVAL, "scales and biases must exist and share x's dtype")
-    K = int(x.shape[-1])
-    M = math.prod(int(d) for d in x.shape[:-1])
-    x2 = _runtime.aligned_contiguous(x.reshape(M, K))
+    if x.dim() == 2:
+        M, K = x.shape
+        x2 = _runtime.aligned_contiguous(x)
+    else:
+        K = int(x.shape[-1])
+        M = math.prod(int(d) for d in x.shape[:-1])
+        x2 = _runtime.aligned_contiguous(x.reshape(M, K))
     return (x2, _runtime.weight_words(w), _runtime.aligned_contiguous(scales),
             _runtime.aligned_contiguous(biases), M, K)
 
@@ -338,7 +342,7 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor,
         x2, wq, s, b, M, K = _prepare(x, w, scales, biases)
         N = int(wq.shape[0])
         y = qmm_launch(x2, wq, s, b, N, group_size, bits, tuning)
-        return y.reshape(*x.shape[:-1], N)
+        return y if x.dim() == 2 else y.reshape(*x.shape[:-1], N)
     return _general(x, w, scales, biases, transpose, int(group_size), int(bits))
 
 
