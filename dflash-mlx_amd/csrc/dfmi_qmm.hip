@@ -215,7 +215,7 @@ __device__ inline void stream_unit_of(int L, int whole, int kp, int xcd_map, int
 // Block nb (of matrix g), K split kpi of kp.  TSB: scales and biases come
 // from g.t, the pair table, one step at a time.  RW = 2: 128-row blocks, two
 // row groups of WV / 2 wavefronts.
-template <typename Tag, int GS, int MT, int WV, int BITS, int SBPC, bool TSB, int RW>
+template <typename Tag, int GS, int MT, int WV, int BITS, int SBPC, int TSB, int RW>
 __device__ __forceinline__ void qmm_stream_body(const StreamArgs& a, const StreamSeg& g, int nb,
                                                 int kpi, int kp, uint32_t tn = 0,
                                                 uint32_t tc = 0) {
@@ -434,11 +434,12 @@ static void plan_tsb(int64_t K, const StreamGeo& geo, int gs, int rw, int kp_for
   } else if (nb < kCUs) {
     const int kp = std::max(1, kCUs / nb);
     p.kp = std::max(kmin, std::min(kp, std::max(1, p.chunks / 2)));
-    // two activation blocks (two stages, one in flight): raise the split
-    // toward two workgroups per CU while every split keeps >= 8 steps
-    // (27B-class down projection at M = 32: 6 splits 23.5 us vs 3 splits
-    // 25.7 us; o: 3 splits 12.0 us, 6 splits 12.7 us)
-    if (mt == 2) p.kp = std::max(p.kp, std::min(2 * kCUs / nb, p.chunks / 8));
+    // two activation blocks: two workgroups per CU where every split keeps
+    // six steps (three stages, M 17 / 32: 12288 x 4096 8 splits 13.2 / 14.6
+    // us, 6 -- one and a half workgroups per CU -- 14.6 / 16.1, 4 14.2 / 14.6;
+    // 17408 x 5120 6 splits 18.2 / 20.2, 3 20.4 / 20.7; 5120 x 5120 3 splits
+    // 10.5 / 10.9, 6 10.7 / 12.1)
+    if (mt == 2 && p.chunks / 6 >= 2 * kCUs / nb) p.kp = std::max(p.kp, 2 * kCUs / nb);
   }
   p.xcd_map = ((nb - p.whole) % 8 == 0) ? 1 : 0;
 }
@@ -591,7 +592,7 @@ static int plan_stream(int64_t M, int64_t K, int64_t N, int gs, int bits,
 // workspace, first needed in the epilogue, last.  (With M, K, N ... after
 // the eight pointers a workgroup waited for one scalar-load round trip
 // before its first DMA.)
-template <typename Tag, int GS, int MT, int WV, int BITS, int SBPC, bool TSB, int RW>
+template <typename Tag, int GS, int MT, int WV, int BITS, int SBPC, int TSB, int RW>
 __global__ __launch_bounds__(64 * WV) void qmm_stream_kernel(
     const uint16_t* x, const uint32_t* w, const uint32_t* t, const uint16_t* s,
     const uint16_t* b, uint32_t p0, int N, int whole, uint32_t tn, uint16_t* y, float* partials,
@@ -611,7 +612,7 @@ __global__ __launch_bounds__(64 * WV) void qmm_stream_kernel(
 
 // Several weight matrices over the same activations (q / k / v, gate / up):
 // their row blocks form one grid.
-template <typename Tag, int GS, int MT, int WV, int BITS, int SBPC, bool TSB, int RW>
+template <typename Tag, int GS, int MT, int WV, int BITS, int SBPC, int TSB, int RW>
 __global__ __launch_bounds__(64 * WV) void qmm_stream_multi_kernel(StreamArgs a, StreamSegs m) {
   int nb, kpi, kpw;
   stream_unit_of(blockIdx.x, a.whole, a.kp, a.xcd_map, nb, kpi, kpw);
@@ -633,7 +634,7 @@ __global__ __launch_bounds__(64 * WV) void qmm_stream_multi_kernel(StreamArgs a,
 // split-K workspace are read from the kernel arguments when the epilogue
 // needs them.  (qmm_stream_multi_kernel instead loads its segment table
 // before the first DMA: ~0.6-0.9 us per launch on MI355X.)
-template <typename Tag, int GS, int MT, int WV, int RW>
+template <typename Tag, int GS, int MT, int WV, int RW, int TSB>
 __global__ __launch_bounds__(64 * WV) void qmm_stream_fused_kernel(
     const uint16_t* x, const uint32_t* t, const uint32_t* w0, const uint32_t* w1,
     const uint32_t* w2, uint32_t p0, uint32_t p1, uint32_t p2, uint16_t* y0, uint16_t* y1,
@@ -658,7 +659,7 @@ __global__ __launch_bounds__(64 * WV) void qmm_stream_fused_kernel(
   g.blk0 = in2 ? b2 : (in1 ? b1 : 0);
   g.t = t;
   const uint32_t tc = in2 ? (uint32_t)(N0 + N1) : (in1 ? (uint32_t)N0 : 0u);
-  qmm_stream_body<Tag, GS, MT, WV, 4, kSbPieces, true, RW>(
+  qmm_stream_body<Tag, GS, MT, WV, 4, kSbPieces, TSB, RW>(
       StreamArgs{x, partials, counters, M, chunks * 256, chunks, kp, n_blocks, xcd_map, pstride,
                  whole},
       g, nb, kpi, kpw, (uint32_t)(N0 + N1 + N2), tc);
@@ -683,7 +684,7 @@ static bool segs_have_pairs(const StreamSegs& m) {
   return true;
 }
 
-template <typename Tag, int GS, int MT, int WV, int BITS, bool TSB, int RW>
+template <typename Tag, int GS, int MT, int WV, int BITS, int TSB, int RW>
 static void launch_stream_k(const StreamPlan& p, hipStream_t st, const StreamArgs& a,
                             const StreamSegs& m) {
   constexpr int SBPC = BITS == 8 && WV == 8 ? 8 : kSbPieces;  // = stream_sb_pieces(BITS, WV)
@@ -704,7 +705,8 @@ static void launch_stream_k(const StreamPlan& p, hipStream_t st, const StreamArg
                             ((uint32_t)a.chunks << 16);
         const uint32_t p1 = (uint32_t)a.whole | ((uint32_t)(m.nseg > 2 ? m.seg[2].N : 0) << 16);
         const uint32_t p2 = (uint32_t)m.seg[0].N | ((uint32_t)m.seg[1].N << 16);
-        hipLaunchKernelGGL((qmm_stream_fused_kernel<Tag, GS, MT, WV, RW>), dim3(p.grid_x),
+        hipLaunchKernelGGL((qmm_stream_fused_kernel<Tag, GS, MT, WV, RW, TSB>),
+                           dim3(p.grid_x),
                            dim3(64 * WV), lds, st, a.x, m.fused, m.seg[0].w, m.seg[1].w,
                            m.nseg > 2 ? m.seg[2].w : m.seg[1].w, p0, p1, p2, m.seg[0].y,
                            m.seg[1].y, m.nseg > 2 ? m.seg[2].y : m.seg[1].y, a.counters,
@@ -727,17 +729,23 @@ static void launch_stream_t(const StreamPlan& p, hipStream_t st, const StreamArg
                             const StreamSegs& m) {
   if constexpr (BITS == 4 && GS >= 64 && MT == 1) {
     if (p.tsb && p.rw == 2 && WV == 8) {
-      launch_stream_k<Tag, GS, MT, 8, BITS, true, 2>(p, st, a, m);
+      launch_stream_k<Tag, GS, MT, 8, BITS, 1, 2>(p, st, a, m);
       return;
     }
   }
   if constexpr (BITS == 4 && GS >= 64 && WV == 4) {
     if (p.tsb && p.rw == 1 && segs_have_pairs(m)) {
-      launch_stream_k<Tag, GS, MT, WV, BITS, true, 1>(p, st, a, m);
+      if constexpr (MT == 2) {
+        if (p.grid_x <= 2 * kCUs) {  // no third workgroup per CU to lose
+          launch_stream_k<Tag, GS, MT, WV, BITS, 2, 1>(p, st, a, m);
+          return;
+        }
+      }
+      launch_stream_k<Tag, GS, MT, WV, BITS, 1, 1>(p, st, a, m);
       return;
     }
   }
-  launch_stream_k<Tag, GS, MT, WV, BITS, false, 1>(p, st, a, m);
+  launch_stream_k<Tag, GS, MT, WV, BITS, 0, 1>(p, st, a, m);
 }
 
 template <typename Tag, int GS, int BITS>
@@ -772,20 +780,32 @@ static void allow_lds_t() {
   constexpr int SBPC = BITS == 8 && WV == 8 ? 8 : kSbPieces;
   constexpr int lds = Stream<Tag, GS, MT, WV, SBPC, BITS>::LDS_BYTES;
   (void)hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&qmm_stream_kernel<Tag, GS, MT, WV, BITS, SBPC, false, 1>),
+      reinterpret_cast<const void*>(&qmm_stream_kernel<Tag, GS, MT, WV, BITS, SBPC, 0, 1>),
       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   (void)hipFuncSetAttribute(
       reinterpret_cast<const void*>(
-          &qmm_stream_multi_kernel<Tag, GS, MT, WV, BITS, SBPC, false, 1>),
+          &qmm_stream_multi_kernel<Tag, GS, MT, WV, BITS, SBPC, 0, 1>),
       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  if constexpr (BITS == 4 && GS >= 64 && MT == 1 && WV == 8) {
-    constexpr int lds2 = Stream<Tag, GS, MT, 8, kSbPieces, 4, 2, true>::LDS_BYTES;
+  if constexpr (BITS == 4 && GS >= 64 && MT == 2) {
+    constexpr int lds2 = Stream<Tag, GS, MT, WV, SBPC, 4, 1, 2>::LDS_BYTES;
     (void)hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&qmm_stream_kernel<Tag, GS, 1, 8, 4, kSbPieces, true, 2>),
+        reinterpret_cast<const void*>(&qmm_stream_kernel<Tag, GS, MT, WV, 4, SBPC, 2, 1>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, lds2);
+    (void)hipFuncSetAttribute(
+        reinterpret_cast<const void*>(&qmm_stream_multi_kernel<Tag, GS, MT, WV, 4, SBPC, 2, 1>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, lds2);
+    (void)hipFuncSetAttribute(
+        reinterpret_cast<const void*>(&qmm_stream_fused_kernel<Tag, GS, MT, WV, 1, 2>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, lds2);
+  }
+  if constexpr (BITS == 4 && GS >= 64 && MT == 1 && WV == 8) {
+    constexpr int lds2 = Stream<Tag, GS, MT, 8, kSbPieces, 4, 2, 1>::LDS_BYTES;
+    (void)hipFuncSetAttribute(
+        reinterpret_cast<const void*>(&qmm_stream_kernel<Tag, GS, 1, 8, 4, kSbPieces, 1, 2>),
         hipFuncAttributeMaxDynamicSharedMemorySize, lds2);
     (void)hipFuncSetAttribute(
         reinterpret_cast<const void*>(
-            &qmm_stream_multi_kernel<Tag, GS, 1, 8, 4, kSbPieces, true, 2>),
+            &qmm_stream_multi_kernel<Tag, GS, 1, 8, 4, kSbPieces, 1, 2>),
         hipFuncAttributeMaxDynamicSharedMemorySize, lds2);
   }
 }

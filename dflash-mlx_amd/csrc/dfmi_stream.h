@@ -138,9 +138,15 @@ __device__ inline uint32_t opaque(uint32_t v) {
 // high half; dfmi_sb_pairs builds it): 64 GPC rows x 4 bytes per 64-row block
 // and step, contiguous, so whole-line requests with no window in LDS (51 KB
 // instead of 80 KB with 4 wavefronts: three workgroups per CU).  The
-// arithmetic is the window path's, operation for operation.
+// arithmetic is the window path's, operation for operation.  TSB = 2: the same
+// with a third stage at two activation blocks (75 KB, two workgroups per CU),
+// for grids of at most two workgroups per CU (M = 17 / 32: gs 64 5120 x 5120
+// 11.1 / 11.4 -> 10.3 / 10.7 us, 5120 x 7168 13.3 / 13.5 -> 12.3 / 12.5, 17408
+// x 5120 17.8 / 20.2 -> 18.3 / 20.4; gs 128 12288 x 4096, with its split, 14.5
+// / 15.8 -> 13.4 / 14.8).  A larger grid keeps its third workgroup per CU:
+// 4096 x 24576, 768 workgroups, 18.8 us, in three stages 23.8.
 template <typename Tag, int GS, int MT, int WV, int SBPC = kSbPieces, int BITS = 4, int RW = 1,
-          bool TSB = false>
+          int TSB = 0>
 struct Stream {
   static constexpr int NT = kStreamTiles;   // 16-row tiles per wavefront
   static constexpr int KW = WV / RW;        // wavefronts along k
@@ -176,7 +182,7 @@ struct Stream {
   // workgroup per CU) and three with pair streaming (78 KB, two per CU).
   static constexpr int DEPTH =
       RW == 2 ? (TSB ? 3 : 4)
-              : ((MT == 2 && BITS == 4) || (MT == 1 && BITS == 8 && WV == 4) ? 2 : 3);
+              : ((MT == 2 && BITS == 4 && TSB < 2) || (MT == 1 && BITS == 8 && WV == 4) ? 2 : 3);
   // gs >= 64: a lane's two k-blocks take adjacent words (one 8-byte LDS read);
   // gs = 32: k-block j is group 2*wave + j, so the blocks stay group-pure.
   static constexpr bool PAIR = GS >= 64;
