@@ -867,8 +867,9 @@ static int validate_qmm(int x_dtype, int64_t M, int64_t K, int64_t N, int gs, in
 using namespace dfmi;
 
 // Automatic choice (measured on MI355X): the streaming kernel is faster on
-// every shape it takes; the general kernel covers the rest (M > 32, K not a
-// multiple of 256 or of 8 groups, weights over 2 GiB).
+// every shape it takes; beyond 32 rows qmm_gemm_kernel (use_gemm), and the
+// general kernel covers the rest (K not a multiple of 256 or of 8 groups,
+// weights over 2 GiB).
 static bool use_stream(int64_t M, int64_t K, int64_t N, int gs, int bits,
                        const dfmi_qmm_tuning* tune) {
   const int path = tune ? tune->path : 0;
@@ -1487,7 +1488,7 @@ extern "C" int dfmi_qmm_prepare(int x_dtype, const dfmi_qmm_segment* segs, int n
   } else {
     // outside the streaming kernel: the shared-activation entry point's own
     // route at each call (a pair table in a wider one is not passed: the
-    // plans it would serve are all streaming)
+    // call builds its own where it reads one)
     for (int i = 0; i < nseg; ++i) {
       r->segs[i] = segs[i];
       r->segs[i].y = nullptr;

@@ -251,11 +251,11 @@ class _VerifyState:
 
     def launch(self, x: torch.Tensor, m: int, st: int) -> torch.Tensor:
         """This module's own launch on x: [m, N]."""
-        x2 = x.reshape(m, self.K)
+        x2 = x if x.dim() == 2 else x.reshape(m, self.K)
         if not x2.is_contiguous() or x2.data_ptr() & 15:
             x2 = _runtime.aligned_contiguous(x2)
         rec = self.recs.get((m, st, x.dtype)) or self.record(m, st, x)
-        y = torch.empty((m, self.N), dtype=x.dtype, device=x.device)
+        y = x2.new_empty((m, self.N))
         rec.run(x2, (y,), st)
         return y
 
@@ -316,7 +316,8 @@ def _build_dispatch(obj: VerifyQuantizedLinear, *, enable_qmm: Optional[bool] = 
                     y = grp.product(state.gidx, x, m, st) if grp is not None else None
                     if y is None:
                         y = state.launch(x, m, st)
-                y = y.view(*shp[:-1], N)
+                if len(shp) != 2:
+                    y = y.view(*shp[:-1], N)
             elif (x.dtype == sdt and x.is_cuda and m > 32 and kx == K and mode == "affine"
                   and (t := state.current_table(obj)) is not None):
                 # many rows: the stock route, with the table the module holds,
@@ -500,24 +501,25 @@ class SiblingGroup:
         # (a captured launch computes nothing until its graph is replayed)
         where = (st, torch.cuda.is_current_stream_capturing()) if many else st
         pending = self._pending
-        if pending is not None and pending[0] is x and pending[1] == x._version \
-                and pending[2] == where:
-            y = pending[3].pop(idx, None)
-            if y is not None:
-                self._miss[idx] = 0
-                if not pending[3] and self._pending is pending:
-                    self._pending = None  # every output taken: let the input go
-                if pending[4] is None or pending[4][idx] == self.states[idx].w._version:
-                    return y
+        if pending is not None:
+            held, ver, there, ys, vers = pending
+            if held is x and ver == x._version and there == where:
+                y = ys.pop(idx, None)
+                if y is not None:
+                    self._miss[idx] = 0
+                    if not ys:
+                        self._pending = None  # every output taken: let the input go
+                    if vers is None or vers[idx] == self.states[idx].w._version:
+                        return y
         active = self.active
         if idx not in active:
             return None
         if many and not self._takes_many(active):
             return None
-        if pending is not None and pending[3]:  # members that did not take their output
+        if pending is not None and ys:  # members that did not take their output
             keep = []
             for j in active:
-                if j in pending[3]:
+                if j in ys:
                     self._miss[j] += 1
                 if self._miss[j] < 2:
                     keep.append(j)
@@ -525,11 +527,10 @@ class SiblingGroup:
             self._pending = None
             if idx not in active or (many and not self._takes_many(active)):
                 return None
-        x2 = x.reshape(m, int(x.shape[-1]))
+        x2 = x if x.dim() == 2 else x.reshape(m, int(x.shape[-1]))
         if not x2.is_contiguous() or x2.data_ptr() & 15:
             x2 = _runtime.aligned_contiguous(x2)
-        outs = [torch.empty((m, self.states[j].N), dtype=x.dtype, device=x.device)
-                for j in active]
+        outs = [x2.new_empty((m, self.states[j].N)) for j in active]
         vers = None
         if many:
             first = self.states[0]

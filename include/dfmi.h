@@ -144,7 +144,10 @@ int dfmi_qmm_general(const void *x, int x_dtype, const uint32_t *w_q, const void
  * holding a scale / bias window in LDS, so three workgroups share a CU.  The
  * launch plan does not depend on sb_pairs: the result is bit-identical to
  * dfmi_qmm_affine_ex (tuning included) on the same inputs; sb_pairs may be
- * NULL.
+ * NULL.  At M > 32 the workspace is optional: with dfmi_qmm_workspace_bytes
+ * bytes of it the same holds (without a table the call builds one there);
+ * with less, K is split less or not at all, and without workspace and table
+ * the general kernel runs, each within fp32 summation order.
  */
 int dfmi_qmm_affine_pairs(const void *x, int x_dtype, const uint32_t *w_q, const void *scales,
                           const void *biases, const uint32_t *sb_pairs, void *y, int64_t M,

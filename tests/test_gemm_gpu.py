@@ -157,6 +157,15 @@ def test_matrices_in_one_launch(dev, M, K, Ns, gs, bits, dtype):
         bits, None, 0, _runtime.stream_ptr(x.device))
     assert rc == _lib.DFMI_OK
     check(outs)
+    ns = (ctypes.c_int64 * len(mats))(*Ns)
+    need = int(_lib.load().dfmi_qmm_multi_workspace_bytes(M, K, ns, len(mats), gs, bits))
+    ws, ws_bytes = _runtime.workspace(x.device, need)
+    for y in outs:
+        y.fill_(float("nan"))
+    rc = _lib.load().dfmi_qmm_affine_multi(  # tables into the workspace, for the call
+        x.data_ptr(), _runtime.dtype_code(x.dtype), segs, len(mats), M, K, gs, bits, ws, ws_bytes,
+        _runtime.stream_ptr(x.device))
+    assert rc == _lib.DFMI_OK and all(torch.equal(a, b) for a, b in zip(one, outs))
 
 
 def test_many_rows_in_inference_mode(dev):
