@@ -102,14 +102,6 @@ class _WorkspaceCache:
         self.get(device, nbytes, kind)
 
 
-    def held(self, device: torch.device, kind: str = "qmm") -> Optional[torch.Tensor]:
-        """This stream's buffer as it is, or None."""
-        key = (device.index if device.index is not None else torch.cuda.current_device(),
-               stream_ptr(device), kind)
-        with self._lock:
-            return self._bufs.get(key)
-
-
 WORKSPACES = _WorkspaceCache()
 
 
@@ -121,24 +113,31 @@ def workspace(device: torch.device, nbytes: int, kind: str = "qmm") -> tuple[int
     return aligned, buf.numel() - (aligned - base)
 
 
-def optional_workspace(device: torch.device, nbytes: int, kind: str = "qmm") -> tuple[int, int]:
-    """:func:`workspace` for a call that also runs with less: while a graph is
-    being captured, when nothing may grow, what the stream holds already (or
-    (0, 0))."""
-    if torch.cuda.is_current_stream_capturing():
-        buf = WORKSPACES.held(device, kind)
-        if buf is None:
-            return 0, 0
-        base = buf.data_ptr()
-        aligned = (base + 255) // 256 * 256
-        return aligned, buf.numel() - (aligned - base)
-    return workspace(device, nbytes, kind)
+def call_scratch(device: torch.device, nbytes: int) -> Optional[torch.Tensor]:
+    """Scratch of one call (None: it needs none).  For a call that enqueues
+    several kernels and passes data between them: another thread's call on the
+    same stream may be enqueued between two of them, so they share no buffer.
+    From torch's stream-ordered allocator (during capture the graph's own
+    pool), contents free; the caller keeps it until the call has returned."""
+    return torch.empty(int(nbytes), dtype=torch.uint8, device=device) if nbytes else None
 
 
 def many_rows(M: int) -> bool:
     """Row counts above the streaming kernels' (``qmm_gemm_kernel``): the
     launch reads a pair table at every group size, bit width and K."""
     return int(M) > 32
+
+
+def launch_space(M: int, device: torch.device, nbytes: int):
+    """(pointer, usable bytes, what keeps them) of a matmul call over M rows:
+    this stream's workspace, or beyond 32 rows, where the call is several
+    kernels, scratch of its own."""
+    if not nbytes:
+        return 0, 0, None
+    if many_rows(M):
+        scratch = call_scratch(device, nbytes)
+        return scratch.data_ptr(), scratch.numel(), scratch
+    return (*workspace(device, nbytes), None)
 
 
 def pair_shape(M: int, K: int, N: int, group_size: int, bits: int) -> bool:

@@ -18,6 +18,11 @@ void set_error(const char* fmt, ...) {
   g_error.assign(buf);
 }
 
+std::mutex& launch_order() {
+  static std::mutex m;
+  return m;
+}
+
 }  // namespace dfmi
 
 extern "C" const char* dfmi_version(void) { return "dfmi 0.1.0 gfx950"; }

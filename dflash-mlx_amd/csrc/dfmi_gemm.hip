@@ -124,6 +124,8 @@ static size_t gemm_space(void* workspace, size_t bytes, char*& ws) {
 int gemm_launch(const void* x, int x_dtype, const dfmi_qmm_segment* segs, int nseg,
                 const uint32_t* fused, int64_t pair_stride, int64_t M, int64_t K, int gs,
                 int bits, void* workspace, size_t workspace_bytes, hipStream_t st) {
+  // (tables, product and split sum pass data through the workspace)
+  std::lock_guard<std::mutex> order(launch_order());
   char* ws;
   size_t left = gemm_space(workspace, workspace_bytes, ws);
   // matrices without a table: theirs into the workspace, for this call

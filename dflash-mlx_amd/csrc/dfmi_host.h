@@ -6,6 +6,7 @@
 
 #include <cstdarg>
 #include <cstdio>
+#include <mutex>
 
 #include "../../include/dfmi.h"
 
@@ -13,6 +14,11 @@ namespace dfmi {
 
 // Thread-local error message (dfmi_last_error).
 void set_error(const char* fmt, ...) __attribute__((format(printf, 1, 2)));
+
+// Held while a call enqueues several kernels that pass data through its
+// workspace: another thread may use that workspace on the same stream, where
+// the stream orders single kernels only.
+std::mutex& launch_order();
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 

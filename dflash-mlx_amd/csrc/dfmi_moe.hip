@@ -1205,6 +1205,8 @@ static int gather_common(const void* x, int x_dtype, int64_t x_rows, const uint3
   a.ws_partials =
       ws_ok ? reinterpret_cast<float*>(static_cast<char*>(workspace) + kMoeWsCounterBytes) : nullptr;
   hipStream_t st = static_cast<hipStream_t>(stream);
+  std::unique_lock<std::mutex> order(launch_order(), std::defer_lock);
+  if (ws_ok && !segs) order.lock();  // (with segs: dfmi_switch_glu holds it)
   // pair-streaming persistent loop (a pair table given): whole 256-k steps,
   // 128-row units, two workgroups per CU, the pair ids in 16-bit LDS tables.
   if (pairs && aligned16(pairs) && moe_stream_eligible(x_rows, P, K, N, E, group_size, glu)) {
@@ -1468,6 +1470,7 @@ extern "C" int dfmi_switch_glu(const void* x, int x_dtype, int64_t T, const void
   int32_t* rhs = order + switch_glu_ints(P);
   int32_t* segs = rhs + switch_glu_ints(P);
   hipStream_t st = static_cast<hipStream_t>(stream);
+  std::lock_guard<std::mutex> launches(launch_order());
   rc = moe_sort_launch(inds, inds_bytes, (int)P, (int)E, order, rhs, segs, st);
   if (rc != DFMI_OK) return rc;
   rc = gather_common(x, x_dtype, T, wg_q, g_scales, g_biases, wu_q, u_scales, u_biases, order, rhs,

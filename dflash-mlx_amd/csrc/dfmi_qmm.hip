@@ -956,6 +956,8 @@ static int prepare_streaming(int x_dtype, const StreamSegs& segs, int64_t M, int
 static int run_streaming(const StreamLaunch& L, const void* x, hipStream_t st) {
   StreamArgs a = L.a;
   a.x = static_cast<const uint16_t*>(x);
+  std::unique_lock<std::mutex> order(launch_order(), std::defer_lock);
+  if (a.partials) order.lock();  // (where gemm_launch may keep its own)
   if (L.x_dtype == DFMI_BF16) launch_stream<BF16>(L.gs, L.p, st, a, L.m);
   else launch_stream<F16>(L.gs, L.p, st, a, L.m);
   return check_launch(L.m.nseg == 1 ? "dfmi_qmm_affine" : "dfmi_qmm_affine_multi");

@@ -78,12 +78,26 @@ def _pairs_ptr(pairs: Optional[torch.Tensor], scales: torch.Tensor, biases: torc
     return table.data_ptr() if table is not None else None
 
 
-def _workspace(lib, device: torch.device, table_ptr):
-    """The stream's gather workspace (tail-split counters and partials), only
-    with a pair table (the plain main loops take none)."""
+def _stream_table(x_rows: int, P: int, K: int, N: int, E: int) -> bool:
+    """Gathers with a pair table of few pairs: one kernel (``moe_stream_kernel``,
+    mirrors the library's rule).  The others are the segment kernel and
+    ``moe_gemm_kernel``."""
+    return (P <= 256 and x_rows <= 32767 and E < 65535 and x_rows * K < 1 << 30
+            and N * K < 1 << 32 and P * N < 1 << 30)
+
+
+def _space(lib, device: torch.device, table_ptr, few: bool):
+    """(pointer, bytes, what keeps them) of a gather's workspace, only with a
+    pair table (the plain main loops take none): the stream's (tail-split
+    counters and partials), or with many pairs scratch of the call's own (its
+    segment table)."""
     if table_ptr is None:
-        return None, 0
-    return _runtime.workspace(device, int(lib.dfmi_gather_workspace_bytes()), kind="gather")
+        return None, 0, None
+    need = int(lib.dfmi_gather_workspace_bytes())
+    if few:
+        return (*_runtime.workspace(device, need, kind="gather"), None)
+    scratch = _runtime.call_scratch(device, need)
+    return scratch.data_ptr(), need, scratch
 
 
 def gather_qmm(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
@@ -116,7 +130,8 @@ def gather_qmm(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: t
     y = torch.empty((P, N), dtype=x.dtype, device=x.device)
     tp = _pairs_ptr(pairs, scales, biases, None, K, N, group_size, bits, use_pairs)
     lib = _lib.load()
-    ws, ws_bytes = _workspace(lib, x.device, tp)
+    few = _stream_table(int(x2.shape[0]), P, K, N, E)
+    ws, ws_bytes, _scratch = _space(lib, x.device, tp, few)
     _lib.check(lib.dfmi_gather_qmm_affine_pairs(
         x2.data_ptr(), _runtime.dtype_code(x.dtype), int(x2.shape[0]), w.data_ptr(),
         scales.data_ptr(), biases.data_ptr(), tp, lhs.data_ptr() if lhs is not None else None,
@@ -147,7 +162,8 @@ def gather_swiglu(x: torch.Tensor, gate: Triple, up: Triple, rhs_indices: torch.
     h = torch.empty((P, N), dtype=x.dtype, device=x.device)
     tp = _pairs_ptr(pairs, sg, bg, (su, bu), K, N, group_size, bits, use_pairs)
     lib = _lib.load()
-    ws, ws_bytes = _workspace(lib, x.device, tp)
+    few = _stream_table(int(x2.shape[0]), P, K, N, Eg)
+    ws, ws_bytes, _scratch = _space(lib, x.device, tp, few)
     _lib.check(lib.dfmi_gather_qmm_swiglu_pairs(
         x2.data_ptr(), _runtime.dtype_code(x.dtype), int(x2.shape[0]), wg.data_ptr(),
         sg.data_ptr(), bg.data_ptr(), wu.data_ptr(), su.data_ptr(), bu.data_ptr(), tp,
@@ -192,8 +208,8 @@ _SORT_MAX_EXPERTS = 1023  # of dfmi_switch_glu
 
 def _switch_glu(x, inds, gate: Triple, up: Triple, down: Triple, group_size: int, bits: int):
     """``dfmi_switch_glu``: sort, both gathers and the pair order in one call.
-    None where it does not apply: x or down of other shapes than one layer's,
-    or a graph capture before the stream has the workspaces."""
+    None where it does not apply: x or down of other shapes than one layer's.
+    The pair order lies in scratch of the call's own."""
     _runtime.require_device(x, "x")
     dev = x.device
     T, k = int(inds.shape[0]), int(inds.shape[1])
@@ -209,20 +225,19 @@ def _switch_glu(x, inds, gate: Triple, up: Triple, down: Triple, group_size: int
     ids = inds.contiguous()
     P = T * k
     lib = _lib.load()
-    need = int(lib.dfmi_switch_glu_workspace_bytes(P))
-    ws, ws_bytes = _runtime.optional_workspace(dev, need, kind="moe_sort")
-    if ws_bytes < need:
-        return None
+    scratch = _runtime.call_scratch(dev, lib.dfmi_switch_glu_workspace_bytes(P))
     h = torch.empty((P, I), dtype=x.dtype, device=dev)
     y = torch.empty((P, D), dtype=x.dtype, device=dev)
     tg = _pairs_ptr(None, sg, bg, (su, bu), D, I, group_size, bits, True)
     td = _pairs_ptr(None, sd, bd, None, I, D, group_size, bits, True)
-    gws, gws_bytes = _workspace(lib, dev, tg or td)
+    few = _stream_table(T, P, D, I, E) and _stream_table(P, P, I, D, E)
+    gws, gws_bytes, _gather = _space(lib, dev, (tg or td) if few else None, few)
     _lib.check(lib.dfmi_switch_glu(
         x2.data_ptr(), _runtime.dtype_code(x.dtype), T, ids.data_ptr(), ids.element_size(), k,
         wg.data_ptr(), sg.data_ptr(), bg.data_ptr(), wu.data_ptr(), su.data_ptr(), bu.data_ptr(),
         wd.data_ptr(), sd.data_ptr(), bd.data_ptr(), tg, td, h.data_ptr(), y.data_ptr(), D, I, E,
-        int(group_size), int(bits), ws, ws_bytes, gws, gws_bytes, _runtime.stream_ptr(dev)),
+        int(group_size), int(bits), scratch.data_ptr(), scratch.numel(), gws, gws_bytes,
+        _runtime.stream_ptr(dev)),
         "dfmi_switch_glu")
     return h, y
 

@@ -142,8 +142,7 @@ def qmm_launch(x2: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: 
     y = out if out is not None else torch.empty((M, N), dtype=x2.dtype, device=dev)
     tptr = ctypes.byref(tuning) if tuning is not None else None
     need = int(lib.dfmi_qmm_workspace_bytes_ex(M, K, N, int(group_size), int(bits), tptr))
-    space = _runtime.optional_workspace if _runtime.many_rows(M) else _runtime.workspace
-    ws, ws_bytes = space(dev, need) if need else (0, 0)
+    ws, ws_bytes, _scratch = _runtime.launch_space(M, dev, need)
     if pair_stride and tuning is None:
         status = lib.dfmi_qmm_affine_pairs_strided(
             x2.data_ptr(), _runtime.dtype_code(x2.dtype), w.data_ptr(), scales.data_ptr(),
@@ -186,8 +185,7 @@ def qmm_multi_launch(x2: torch.Tensor, mats, group_size: int, bits: int,
         segs[i].sb_pairs = t.data_ptr() if t is not None else 0
     ns = (ctypes.c_int64 * n)(*Ns)
     need = int(lib.dfmi_qmm_multi_workspace_bytes(M, K, ns, n, int(group_size), int(bits)))
-    space = _runtime.optional_workspace if _runtime.many_rows(M) else _runtime.workspace
-    ws, ws_bytes = space(dev, need) if need else (0, 0)
+    ws, ws_bytes, _scratch = _runtime.launch_space(M, dev, need)
     # two or three matrices with tables: the tables side by side, so that the
     # fused kernel starts its first loads without reading a segment table
     # (many rows: the matrix-core kernel takes them apart as well)
@@ -222,8 +220,7 @@ def qmm_fused_launch(x2: torch.Tensor, mats, fused: torch.Tensor, group_size: in
         segs[i].y, segs[i].N = y.data_ptr(), int(w.shape[0])
         ns[i] = int(w.shape[0])
     need = int(lib.dfmi_qmm_multi_workspace_bytes(M, K, ns, n, int(group_size), int(bits)))
-    space = _runtime.optional_workspace if _runtime.many_rows(M) else _runtime.workspace
-    ws, ws_bytes = space(dev, need) if need else (0, 0)
+    ws, ws_bytes, _scratch = _runtime.launch_space(M, dev, need)
     status = lib.dfmi_qmm_affine_multi_fused(
         x2.data_ptr(), _runtime.dtype_code(x2.dtype), segs, n, fused.data_ptr(), M, K,
         int(group_size), int(bits), ws, ws_bytes, _runtime.stream_ptr(dev))
@@ -251,9 +248,10 @@ class LaunchRecord:
     ``sb_stride`` names that table's row length); ``fused``: for 2..4
     matrices, their tables side by side.  The record keeps these tensors and
     the stream's workspace alive while it exists; run it only on the stream
-    it was prepared for (the workspace is that stream's)."""
+    it was prepared for (the workspace is that stream's).  Beyond 32 rows a
+    run is one :func:`qmm_multi_launch`, with scratch of its own."""
 
-    __slots__ = ("_buf", "ptr", "_keep", "M", "Ns", "dtype")
+    __slots__ = ("_buf", "ptr", "_keep", "M", "Ns", "dtype", "_many")
 
     def __init__(self, M: int, K: int, dtype: torch.dtype, dev: torch.device, mats,
                  group_size: int, bits: int, fused: Optional[torch.Tensor] = None,
@@ -283,8 +281,8 @@ class LaunchRecord:
             ns = (ctypes.c_int64 * n)(*Ns)
             need = int(lib.dfmi_qmm_multi_workspace_bytes(M, K, ns, n, int(group_size),
                                                           int(bits)))
-        space = _runtime.optional_workspace if _runtime.many_rows(M) else _runtime.workspace
-        ws, ws_bytes = space(dev, need) if need else (0, 0)
+        many = _runtime.many_rows(M)  # (each run brings scratch of its own)
+        ws, ws_bytes = _runtime.workspace(dev, need) if need and not many else (0, 0)
         buf = ctypes.create_string_buffer(_lib.DFMI_QMM_RECORD_BYTES + 16)
         ptr = (ctypes.addressof(buf) + 15) // 16 * 16
         status = lib.dfmi_qmm_prepare(_runtime.dtype_code(dtype), segs, n,
@@ -295,9 +293,20 @@ class LaunchRecord:
         keep.append(fused)
         self._buf, self.ptr, self._keep = buf, ptr, keep
         self.M, self.Ns, self.dtype = M, Ns, dtype
+        self._many = (([(m[0], m[1], m[2]) for m in mats], int(group_size), int(bits))
+                      if many else None)
 
     def run(self, x2: torch.Tensor, ys, stream: int) -> None:
         """Launch on ``x2 [M, K]`` (contiguous, 16-byte aligned) into ``ys``."""
+        if self._many is not None:
+            dev = x2.device
+            if int(stream) == current_stream(dev.index):
+                qmm_multi_launch(x2, *self._many, outs=ys)
+            else:
+                with torch.cuda.stream(torch.cuda.ExternalStream(int(stream), device=dev) if stream
+                                       else torch.cuda.default_stream(dev)):
+                    qmm_multi_launch(x2, *self._many, outs=ys)
+            return
         p = [y.data_ptr() for y in ys] + [None] * (4 - len(ys))
         status = _lib.load().dfmi_qmm_run(self.ptr, x2.data_ptr(), p[0], p[1], p[2], p[3], stream)
         if status:
@@ -386,8 +395,7 @@ def _general(x, w, scales, biases, transpose: bool, group_size: int, bits: int):
     need = 0
     if transpose and x.dtype == scales.dtype and x.dtype != torch.float32:
         need = int(lib.dfmi_qmm_workspace_bytes(M, K, N, group_size, bits))
-    space = _runtime.optional_workspace if _runtime.many_rows(M) else _runtime.workspace
-    ws, ws_bytes = space(x.device, need) if need else (0, 0)
+    ws, ws_bytes, _scratch = _runtime.launch_space(M, x.device, need)
     status = lib.dfmi_qmm_general(
         x2.data_ptr(), _runtime.dtype_code(x2.dtype), wq.data_ptr(), s.data_ptr(), b.data_ptr(),
         _runtime.dtype_code(s.dtype), y.data_ptr(), M, K, N, group_size, bits, int(bool(transpose)),

@@ -100,6 +100,8 @@ typedef struct dfmi_qmm_tuning {
  * keeps the partial tiles of a K split in it, and the pair table where the
  * call brings none; with less of it the call runs unsplit, or on the general
  * kernel (the sums of another split are in another fp32 order).
+ * A call is one or several kernels; threads may use one workspace on one
+ * stream, the library enqueues each call's kernels together.
  */
 int dfmi_qmm_affine(const void *x, int x_dtype, const uint32_t *w_q, const void *scales,
                     const void *biases, void *y, int64_t M, int64_t K, int64_t N,
@@ -352,17 +354,18 @@ int dfmi_gather_qmm_swiglu(const void *x, int x_dtype, int64_t x_rows,
  * main loop that streams the pairs per 256-k step (128-row work units, two
  * workgroups per CU).  Taken when sb_pairs != NULL (16-byte aligned), gs is
  * 64 or 128, K % 256 == 0, N % 128 == 0 (affine) or N % 64 == 0 (SwiGLU),
- * P <= 256, x_rows <= 32767 and E < 65535; otherwise the call is exactly the
- * plain entry point's.  Same call sites as dfmi_gather_qmm_affine /
+ * P <= 256, x_rows <= 32767 and E < 65535; with more pairs or rows, and the
+ * workspace, 32-row tiles of the matrix-core kernel read the table; otherwise
+ * the call is exactly the plain entry point's.  Same call sites as dfmi_gather_qmm_affine /
  * dfmi_gather_qmm_swiglu (mlx-lm QuantizedSwitchLinear / SwitchGLU, reached
  * from dflash_mlx/engine/target_qwen_gdn.py:865,874), with the per-layer
  * table built once, as the reference's VerifyQuantizedLinear precomputes
  * per-module state (dflash_mlx/verify_linear.py:118-223).
  * workspace (16-byte aligned, dfmi_gather_workspace_bytes() bytes: 4 KiB
  * of counters, zero when first used and left zero by every call, then the
- * pieces' fp32 partials, which need no clearing) lets the units of the last
- * partial round split along K; NULL runs them whole.  Calls that overlap
- * on one workspace race.
+ * pieces' fp32 partials, or beyond 256 pairs the segment table, which need no
+ * clearing) lets the units of the last partial round split along K; NULL runs
+ * them whole.  Calls on different streams that overlap on one workspace race.
  */
 int dfmi_gather_qmm_affine_pairs(const void *x, int x_dtype, int64_t x_rows,
                                  const uint32_t *w_q, const void *scales, const void *biases,

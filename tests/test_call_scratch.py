@@ -1,0 +1,204 @@
+"""Host side of the calls that enqueue several kernels and pass data between
+them through scratch (more than 32 rows, more than 256 routed pairs, the expert
+sort): two calls in flight on one stream share no byte of it.  CPU only: a
+stand-in library records the scratch each call brings and holds the first call
+inside the library until the second one has been there."""
+
+from __future__ import annotations
+
+import threading
+
+import pytest
+import torch
+
+from dflash_mlx_amd import _lib, _runtime, moe, verify_qmm as vq
+
+
+class _Library:
+    """Answers as libdfmi does, launching nothing."""
+
+    def __init__(self, entry, ws):
+        self.entry, self.ws = entry, ws  # entry point looked at; positions of (ptr, bytes) pairs
+        self.seen = []
+        self.second = threading.Event()
+
+    def __getattr__(self, name):
+        def call(*args):
+            if name.endswith("workspace_bytes") or name.endswith("workspace_bytes_ex"):
+                return 65536 + 4096
+            if name == self.entry:
+                self.seen.append([(args[i], args[i + 1]) for i in self.ws])
+                if len(self.seen) == 1:
+                    self.second.wait(10)
+                else:
+                    self.second.set()
+            return _lib.DFMI_OK
+        return call
+
+
+@pytest.fixture
+def library(monkeypatch):
+    def use(entry, ws):
+        lib = _Library(entry, ws)
+        monkeypatch.setattr(_lib, "load", lambda: lib)
+        return lib
+
+    monkeypatch.setattr(_runtime, "require_device", lambda t, name: None)
+    monkeypatch.setattr(_runtime, "_raw_stream", lambda i: 0)
+    monkeypatch.setattr(vq, "_raw_stream", lambda i: 0)
+    monkeypatch.setattr(_runtime, "stream_ptr", lambda dev: 0)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(_runtime.PAIRS, "get", lambda *a, **k: torch.zeros(1))
+    monkeypatch.setattr(_runtime, "WORKSPACES", _runtime._WorkspaceCache())
+    return use
+
+
+def _weights(N, K, gs=64, lead=()):
+    bf = torch.bfloat16
+    return (torch.zeros((*lead, N, K // 8), dtype=torch.int32),
+            torch.zeros((*lead, N, K // gs), dtype=bf), torch.zeros((*lead, N, K // gs), dtype=bf))
+
+
+def _two_at_once(lib, call):
+    first = threading.Thread(target=call)
+    first.start()
+    while not lib.seen:
+        first.join(0.01)
+        assert first.is_alive() or lib.seen
+    call()
+    first.join()
+    a, b = lib.seen
+    for (pa, na), (pb, nb) in zip(a, b):
+        assert pa and pb and na and nb
+        assert pa + na <= pb or pb + nb <= pa, "two calls in flight share scratch"
+
+
+@pytest.mark.parametrize("route", ["single", "siblings", "general", "record"])
+def test_many_rows(library, route):
+    x, w = torch.zeros((40, 256), dtype=torch.bfloat16), _weights(128, 256)
+    if route == "single":
+        lib = library("dfmi_qmm_affine_pairs", (12,))
+        _two_at_once(lib, lambda: vq.quantized_matmul(x, *w))
+    elif route == "siblings":
+        lib = library("dfmi_qmm_affine_multi", (8,))
+        _two_at_once(lib, lambda: vq.quantized_matmul_multi(x, [w, w]))
+    elif route == "general":
+        lib = library("dfmi_qmm_general", (13,))
+        _two_at_once(lib, lambda: vq._general(x, *w, True, 64, 4))
+    else:
+        lib = library("dfmi_qmm_affine_multi", (8,))
+        rec = vq.LaunchRecord(40, 256, x.dtype, x.device, [w], 64, 4)
+        _two_at_once(lib, lambda: rec.run(x, [torch.empty((40, 128), dtype=x.dtype)], 0))
+
+
+def test_many_pairs(library):
+    E, D = 4, 256
+    w = _weights(128, D, lead=(E,))
+    x = torch.zeros((300, D), dtype=torch.bfloat16)
+    ids = torch.zeros(300, dtype=torch.int32)
+    lib = library("dfmi_gather_qmm_affine_pairs", (16,))
+    _two_at_once(lib, lambda: moe.gather_qmm(x, *w, ids))
+    lib = library("dfmi_gather_qmm_swiglu_pairs", (19,))
+    _two_at_once(lib, lambda: moe.gather_swiglu(x, w, w, ids))
+
+
+def test_expert_sort(library):
+    E, D, I = 4, 256, 128
+    gate, down = _weights(I, D, lead=(E,)), _weights(D, I, lead=(E,))
+    x = torch.zeros((16, D), dtype=torch.bfloat16)
+    ids = torch.zeros((16, 8), dtype=torch.int32)
+    lib = library("dfmi_switch_glu", (24,))
+    _two_at_once(lib, lambda: moe._switch_glu(x, ids, gate, gate, down, 64, 4))
+
+
+def _from_two_threads(calls, check):
+    errors = []
+
+    def work(i):
+        try:
+            for _ in range(60):
+                check(i, calls[i]())
+        except Exception as exc:  # reported by the main thread
+            errors.append(exc)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors[0]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shared", [False, True])
+def test_threads_on_one_stream(dev, shared):
+    """K splits (product, then sum) from two threads on one stream, through
+    the operator and through the C ABI with one workspace for both: each call
+    has its own result."""
+    M, K, Ns, gs = 40, 4096, (256, 512), 64
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(2)
+
+    def rand(*shape):
+        return torch.randn(shape, generator=gen, device=dev).to(torch.bfloat16)
+
+    xs = [rand(M, K) for _ in Ns]
+    mats = [(torch.randint(-2 ** 31, 2 ** 31 - 1, (N, K // 8), generator=gen, device=dev,
+                           dtype=torch.int32), rand(N, K // gs), rand(N, K // gs)) for N in Ns]
+    want = [vq.quantized_matmul(x, *w, group_size=gs) for x, w in zip(xs, mats)]
+    lib = _lib.load()
+    need = max(int(lib.dfmi_qmm_workspace_bytes(M, K, N, gs, 4)) for N in Ns)
+    ws = torch.zeros(need, dtype=torch.uint8, device=dev)
+    st = _runtime.stream_ptr(dev)
+    torch.cuda.synchronize()
+
+    def through_abi(i):
+        y = torch.empty((M, Ns[i]), dtype=torch.bfloat16, device=dev)
+        w, s, b = mats[i]
+        rc = lib.dfmi_qmm_affine(xs[i].data_ptr(), _lib.DFMI_BF16, w.data_ptr(), s.data_ptr(),
+                                 b.data_ptr(), y.data_ptr(), M, K, Ns[i], gs, 4, ws.data_ptr(),
+                                 int(lib.dfmi_qmm_workspace_bytes(M, K, Ns[i], gs, 4)), st)
+        assert rc == _lib.DFMI_OK
+        return y
+
+    def through_operator(i):
+        return vq.quantized_matmul(xs[i], *mats[i], group_size=gs)
+
+    call = through_abi if shared else through_operator
+
+    def check(i, y):
+        torch.cuda.synchronize()
+        assert torch.equal(y, want[i])
+
+    _from_two_threads([lambda i=i: call(i) for i in range(2)], check)
+
+
+@pytest.mark.gpu
+def test_expert_routing_from_two_threads(dev):
+    """The sorted pairs of two threads' SwitchGLU calls on one stream stay
+    apart, with few and many pairs."""
+    from dflash_mlx_amd.quantize import quantize
+
+    E, D, I, gs = 8, 256, 128, 64
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(4)
+
+    def experts(N, K):
+        w = torch.randn((E * N, K), generator=gen, device=dev) * 0.05
+        return tuple(t.reshape(E, N, -1) for t in quantize(w, gs, 4, torch.bfloat16))
+
+    gate, up, down = experts(I, D), experts(I, D), experts(D, I)
+    args = []
+    for T in (90, 16):
+        x = torch.randn((T, D), generator=gen, device=dev).to(torch.bfloat16)
+        args.append((x, torch.randint(0, E, (T, 4), generator=gen, device=dev)))
+    want = [moe.switch_glu(x, ids, gate, up, down, group_size=gs) for x, ids in args]
+    torch.cuda.synchronize()
+
+    def check(i, got):
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want[i]))
+
+    _from_two_threads([lambda i=i: moe.switch_glu(*args[i], gate, up, down, group_size=gs)
+                       for i in range(2)], check)
