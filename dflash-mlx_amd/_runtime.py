@@ -123,8 +123,8 @@ def call_scratch(device: torch.device, nbytes: int) -> Optional[torch.Tensor]:
 
 
 def many_rows(M: int) -> bool:
-    """Row counts above the streaming kernels' (``qmm_gemm_kernel``): the
-    launch reads a pair table at every group size, bit width and K."""
+    """Row counts above the streaming kernels' (``qmm_gemm_kernel``, which
+    reads a pair table at every group size, bit width and K)."""
     return int(M) > 32
 
 
@@ -227,8 +227,11 @@ class _PairCache:
     update or storage swapped in rebuilds it; inference tensors count no
     versions and get no table).  Nothing is built during graph capture: the caller
     then runs without a table (dense matmuls: the same plan, bit-identical
-    result; gathers: the plain gather's main loop).  ``experts`` selects the
-    routed-expert layout (``dfmi_moe_pairs``; with ``up`` the SwiGLU
+    result; gathers: the plain gather's main loop).  Calls beyond 32 rows or 256
+    pairs take none from here: their tables are built in each call, so that
+    they see every update (also one that counts no version, or that falls
+    between the replays of a graph).  ``experts`` selects the routed-expert
+    layout (``dfmi_moe_pairs``; with ``up`` the SwiGLU
     interleave of two sets)."""
 
     def __init__(self):

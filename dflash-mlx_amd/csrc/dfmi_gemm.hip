@@ -1,5 +1,6 @@
 // Planning and launch of qmm_gemm_kernel (dfmi_gemm.h).
 #include "dfmi_gemm.h"
+#include "dfmi_pairs.h"
 
 #include <algorithm>
 
@@ -141,6 +142,8 @@ int gemm_launch(const void* x, int x_dtype, const dfmi_qmm_segment* segs, int ns
   a.nseg = nseg;
   a.M = (int)M;
   a.K = (int)K;
+  PairArgs build{};
+  build.G = (int)(K / gs);
   for (int i = 0; i < nseg; ++i) {
     const int64_t N = segs[i].N;
     a.w[i] = segs[i].w_q;
@@ -155,13 +158,18 @@ int gemm_launch(const void* x, int x_dtype, const dfmi_qmm_segment* segs, int ns
       a.tn[i] = (uint32_t)(pair_stride ? pair_stride : N);
     } else {
       uint32_t* t = reinterpret_cast<uint32_t*>(ws);
-      const int rc = dfmi_sb_pairs(segs[i].scales, segs[i].biases, x_dtype, N, K / gs, t, st);
-      if (rc != DFMI_OK) return rc;
+      build.seg[build.nseg++] = PairSeg{static_cast<const uint16_t*>(segs[i].scales),
+                                        static_cast<const uint16_t*>(segs[i].biases),
+                                        nullptr, nullptr, t, (int)N, 0};
       a.t[i] = t;
       a.tn[i] = (uint32_t)N;
       ws += table_bytes(K, N, gs);
       left -= table_bytes(K, N, gs);
     }
+  }
+  if (build.nseg > 0) {
+    const int rc = pairs_launch(build, 1, st, "dfmi_qmm_affine (pair tables)");
+    if (rc != DFMI_OK) return rc;
   }
   return gemm_run(a, x_dtype, gs, bits, ws, left, st);
 }

@@ -23,6 +23,7 @@
 #include "dfmi_core.h"
 #include "dfmi_host.h"
 #include "dfmi_moe_gemm.h"
+#include "dfmi_pairs.h"
 #include "dfmi_stream.h"
 
 namespace dfmi {
@@ -1484,38 +1485,7 @@ extern "C" int dfmi_switch_glu(const void* x, int x_dtype, int64_t T, const void
 
 // Pair tables of expert weights: [E][G][N] from one (scales, biases) set, or
 // for the SwiGLU [E][G][2N] interleaving the gate and up sets 32 columns at a
-// time (table column 64 (n / 32) + 32 up + n % 32).  Each workgroup
-// transposes 64 table columns x 64 groups of one expert through LDS.
-__global__ __launch_bounds__(256) void moe_pairs_kernel(const uint16_t* s0, const uint16_t* b0,
-                                                        const uint16_t* s1, const uint16_t* b1,
-                                                        uint32_t* t, int N, int G) {
-  __shared__ uint32_t tile[64][65];
-  const bool glu = s1 != nullptr;
-  const int ntc = glu ? 2 * N : N;
-  const int c0 = blockIdx.x * 64, g0 = blockIdx.y * 64;
-  const int64_t e = blockIdx.z;
-  for (int i = threadIdx.x; i < 64 * 64; i += 256) {
-    const int r = i / 64, gi = i % 64;  // table column c0 + r, group g0 + gi
-    const int c = c0 + r, g = g0 + gi;
-    uint32_t v = 0;
-    if (c < ntc && g < G) {
-      const bool up = glu && (c & 32);
-      const int n = glu ? 32 * (c >> 6) + (c & 31) : c;
-      const int64_t o = (e * N + n) * G + g;
-      const uint16_t sv = up ? s1[o] : s0[o];
-      const uint16_t bv = up ? b1[o] : b0[o];
-      v = (uint32_t)sv | ((uint32_t)bv << 16);
-    }
-    tile[r][gi] = v;
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < 64 * 64; i += 256) {
-    const int gi = i / 64, r = i % 64;
-    const int c = c0 + r, g = g0 + gi;
-    if (c < ntc && g < G) t[(e * G + g) * ntc + c] = tile[r][gi];
-  }
-}
-
+// time.
 extern "C" int dfmi_moe_pairs(const void* scales, const void* biases, const void* up_scales,
                               const void* up_biases, int dtype, int64_t E, int64_t N,
                               int64_t groups, uint32_t* sb_pairs, void* stream) {
@@ -1535,13 +1505,13 @@ extern "C" int dfmi_moe_pairs(const void* scales, const void* biases, const void
     set_error("dfmi_moe_pairs: null pointer");
     return DFMI_EINVAL;
   }
-  const int64_t ntc = glu ? 2 * N : N;
-  const dim3 grid((unsigned)((ntc + 63) / 64), (unsigned)((groups + 63) / 64), (unsigned)E);
-  hipLaunchKernelGGL(moe_pairs_kernel, grid, dim3(256), 0, static_cast<hipStream_t>(stream),
-                     static_cast<const uint16_t*>(scales), static_cast<const uint16_t*>(biases),
+  PairArgs a{};
+  a.seg[0] = PairSeg{static_cast<const uint16_t*>(scales), static_cast<const uint16_t*>(biases),
                      static_cast<const uint16_t*>(up_scales),
-                     static_cast<const uint16_t*>(up_biases), sb_pairs, (int)N, (int)groups);
-  return check_launch("dfmi_moe_pairs");
+                     static_cast<const uint16_t*>(up_biases), sb_pairs, (int)N, 0};
+  a.nseg = 1;
+  a.G = (int)groups;
+  return pairs_launch(a, E, static_cast<hipStream_t>(stream), "dfmi_moe_pairs");
 }
 
 extern "C" int dfmi_moe_combine(const void* y, int y_dtype, const int32_t* y_rows,

@@ -13,6 +13,7 @@
 
 #include "dfmi_core.h"
 #include "dfmi_host.h"
+#include "dfmi_pairs.h"
 #include "dfmi_stream.h"
 
 namespace dfmi {
@@ -1546,31 +1547,7 @@ extern "C" int dfmi_qmm_run(const void* record, const void* x, void* y0, void* y
 
 // ---------------------------------------------------------------------------
 // Pair table of the pair-streaming kernels: pairs[g][n] = scales[n][g] |
-// biases[n][g] << 16 (16-bit values of either activation dtype).  Each
-// workgroup transposes a 64 (rows) x 64 (groups) tile through LDS so that
-// both the reads (along groups) and the writes (along rows) are contiguous.
-__global__ __launch_bounds__(256) void sb_pairs_kernel(const uint16_t* s, const uint16_t* b,
-                                                       uint32_t* t, int N, int G) {
-  __shared__ uint32_t tile[64][65];
-  const int n0 = blockIdx.x * 64, g0 = blockIdx.y * 64;
-  for (int i = threadIdx.x; i < 64 * 64; i += 256) {
-    const int r = i / 64, c = i % 64;  // row n0 + r, group g0 + c
-    const int n = n0 + r, g = g0 + c;
-    uint32_t v = 0;
-    if (n < N && g < G) {
-      const int64_t o = (int64_t)n * G + g;
-      v = (uint32_t)s[o] | ((uint32_t)b[o] << 16);
-    }
-    tile[r][c] = v;
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < 64 * 64; i += 256) {
-    const int c = i / 64, r = i % 64;  // group g0 + c, row n0 + r
-    const int n = n0 + r, g = g0 + c;
-    if (n < N && g < G) t[(int64_t)g * N + n] = tile[r][c];
-  }
-}
-
+// biases[n][g] << 16 (16-bit values of either activation dtype).
 extern "C" int dfmi_sb_pairs(const void* scales, const void* biases, int dtype, int64_t N,
                              int64_t groups, uint32_t* sb_pairs, void* stream) {
   if (dtype != DFMI_BF16 && dtype != DFMI_F16) {
@@ -1587,9 +1564,10 @@ extern "C" int dfmi_sb_pairs(const void* scales, const void* biases, int dtype, 
     set_error("dfmi_sb_pairs: null pointer");
     return DFMI_EINVAL;
   }
-  const dim3 grid((unsigned)((N + 63) / 64), (unsigned)((groups + 63) / 64));
-  hipLaunchKernelGGL(sb_pairs_kernel, grid, dim3(256), 0, static_cast<hipStream_t>(stream),
-                     static_cast<const uint16_t*>(scales), static_cast<const uint16_t*>(biases),
-                     sb_pairs, (int)N, (int)groups);
-  return check_launch("dfmi_sb_pairs");
+  PairArgs a{};
+  a.seg[0] = PairSeg{static_cast<const uint16_t*>(scales), static_cast<const uint16_t*>(biases),
+                     nullptr, nullptr, sb_pairs, (int)N, 0};
+  a.nseg = 1;
+  a.G = (int)groups;
+  return pairs_launch(a, 1, static_cast<hipStream_t>(stream), "dfmi_sb_pairs");
 }

@@ -20,7 +20,7 @@ pass over both weight sets), and the weighted sum is ``dfmi_moe_combine``.
 Where the expert shapes allow (4-bit, gs 64 / 128, K a multiple of 256,
 N a multiple of 128, or 64 for the SwiGLU pair) the
 gathers take the experts' (scale, bias) pair table (``dfmi_moe_pairs``,
-built once per weight set and cached) and the stream's gather workspace, and
+built once per weight set and cached, or beyond 256 pairs in each call) and the stream's gather workspace, and
 run the pair-streaming main loop (``dfmi_gather_qmm_*_pairs``); otherwise,
 and during graph capture before a table exists, the plain entry points.
 """
@@ -56,14 +56,15 @@ def _expert_weights(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
             _runtime.aligned_contiguous(biases))
 
 
-def _pairs_ptr(pairs: Optional[torch.Tensor], scales: torch.Tensor, biases: torch.Tensor,
-               up: Optional[Tuple[torch.Tensor, torch.Tensor]], K: int, N: int,
-               group_size: int, bits: int, use_pairs: bool):
-    """Address of the experts' pair table (``dfmi_moe_pairs`` layout), or None.
+def _pairs_table(pairs: Optional[torch.Tensor], scales: torch.Tensor, biases: torch.Tensor,
+                 up: Optional[Tuple[torch.Tensor, torch.Tensor]], K: int, N: int,
+                 group_size: int, bits: int, use_pairs: bool, few: bool):
+    """The experts' pair table (``dfmi_moe_pairs`` layout), or None.
 
-    An explicit table is checked for shape and device; otherwise the cached
-    table of these scales / biases is used when the shape takes one (built on
-    first use, never during graph capture)."""
+    An explicit table is checked for shape and device; otherwise, where the
+    shape takes one, it is the cached table of these scales / biases (few
+    pairs: built on first use, never during graph capture) or one built for
+    the call from the scales as they are (many pairs)."""
     E, _, G = (int(d) for d in scales.shape)
     cols = 2 * N if up is not None else N
     if pairs is not None:
@@ -71,11 +72,16 @@ def _pairs_ptr(pairs: Optional[torch.Tensor], scales: torch.Tensor, biases: torc
         if (pairs.dtype != torch.int32 or tuple(pairs.shape) != (E, G, cols)
                 or not pairs.is_contiguous()):
             raise ValueError(f"pairs must be a contiguous int32 [{E}, {G}, {cols}] table")
-        return pairs.data_ptr()
+        return pairs
     if not use_pairs or not _runtime.moe_pair_shape(K, N, group_size, bits, up is not None):
         return None
-    table = _runtime.PAIRS.get(scales, biases, up, experts=True)
-    return table.data_ptr() if table is not None else None
+    if few:
+        return _runtime.PAIRS.get(scales, biases, up, experts=True)
+    return _runtime.build_moe_pairs(scales, biases, *(up if up is not None else ()))
+
+
+def _ptr(t: Optional[torch.Tensor]):
+    return t.data_ptr() if t is not None else None
 
 
 def _stream_table(x_rows: int, P: int, K: int, N: int, E: int) -> bool:
@@ -86,12 +92,12 @@ def _stream_table(x_rows: int, P: int, K: int, N: int, E: int) -> bool:
             and N * K < 1 << 32 and P * N < 1 << 30)
 
 
-def _space(lib, device: torch.device, table_ptr, few: bool):
+def _space(lib, device: torch.device, table, few: bool):
     """(pointer, bytes, what keeps them) of a gather's workspace, only with a
     pair table (the plain main loops take none): the stream's (tail-split
     counters and partials), or with many pairs scratch of the call's own (its
     segment table)."""
-    if table_ptr is None:
+    if table is None:
         return None, 0, None
     need = int(lib.dfmi_gather_workspace_bytes())
     if few:
@@ -128,13 +134,13 @@ def gather_qmm(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: t
     if lhs is not None and int(lhs.shape[0]) != P:
         raise ValueError("lhs_indices and rhs_indices must have the same length")
     y = torch.empty((P, N), dtype=x.dtype, device=x.device)
-    tp = _pairs_ptr(pairs, scales, biases, None, K, N, group_size, bits, use_pairs)
-    lib = _lib.load()
     few = _stream_table(int(x2.shape[0]), P, K, N, E)
-    ws, ws_bytes, _scratch = _space(lib, x.device, tp, few)
+    table = _pairs_table(pairs, scales, biases, None, K, N, group_size, bits, use_pairs, few)
+    lib = _lib.load()
+    ws, ws_bytes, _scratch = _space(lib, x.device, table, few)
     _lib.check(lib.dfmi_gather_qmm_affine_pairs(
         x2.data_ptr(), _runtime.dtype_code(x.dtype), int(x2.shape[0]), w.data_ptr(),
-        scales.data_ptr(), biases.data_ptr(), tp, lhs.data_ptr() if lhs is not None else None,
+        scales.data_ptr(), biases.data_ptr(), _ptr(table), lhs.data_ptr() if lhs is not None else None,
         rhs.data_ptr(), y.data_ptr(), P, K, N, E, int(group_size), int(bits), ws, ws_bytes,
         _runtime.stream_ptr(x.device)), "dfmi_gather_qmm_affine_pairs")
     return y
@@ -160,13 +166,13 @@ def gather_swiglu(x: torch.Tensor, gate: Triple, up: Triple, rhs_indices: torch.
     lhs = _indices(lhs_indices, "lhs_indices")
     P = int(rhs.shape[0])
     h = torch.empty((P, N), dtype=x.dtype, device=x.device)
-    tp = _pairs_ptr(pairs, sg, bg, (su, bu), K, N, group_size, bits, use_pairs)
-    lib = _lib.load()
     few = _stream_table(int(x2.shape[0]), P, K, N, Eg)
-    ws, ws_bytes, _scratch = _space(lib, x.device, tp, few)
+    table = _pairs_table(pairs, sg, bg, (su, bu), K, N, group_size, bits, use_pairs, few)
+    lib = _lib.load()
+    ws, ws_bytes, _scratch = _space(lib, x.device, table, few)
     _lib.check(lib.dfmi_gather_qmm_swiglu_pairs(
         x2.data_ptr(), _runtime.dtype_code(x.dtype), int(x2.shape[0]), wg.data_ptr(),
-        sg.data_ptr(), bg.data_ptr(), wu.data_ptr(), su.data_ptr(), bu.data_ptr(), tp,
+        sg.data_ptr(), bg.data_ptr(), wu.data_ptr(), su.data_ptr(), bu.data_ptr(), _ptr(table),
         lhs.data_ptr() if lhs is not None else None, rhs.data_ptr(), h.data_ptr(), P, K, N,
         Eg, int(group_size), int(bits), ws, ws_bytes, _runtime.stream_ptr(x.device)),
         "dfmi_gather_qmm_swiglu_pairs")
@@ -228,14 +234,15 @@ def _switch_glu(x, inds, gate: Triple, up: Triple, down: Triple, group_size: int
     scratch = _runtime.call_scratch(dev, lib.dfmi_switch_glu_workspace_bytes(P))
     h = torch.empty((P, I), dtype=x.dtype, device=dev)
     y = torch.empty((P, D), dtype=x.dtype, device=dev)
-    tg = _pairs_ptr(None, sg, bg, (su, bu), D, I, group_size, bits, True)
-    td = _pairs_ptr(None, sd, bd, None, I, D, group_size, bits, True)
     few = _stream_table(T, P, D, I, E) and _stream_table(P, P, I, D, E)
-    gws, gws_bytes, _gather = _space(lib, dev, (tg or td) if few else None, few)
+    glu = _pairs_table(None, sg, bg, (su, bu), D, I, group_size, bits, True, few)
+    dn = _pairs_table(None, sd, bd, None, I, D, group_size, bits, True, few)
+    gws, gws_bytes, _gather = _space(lib, dev, (glu if glu is not None else dn) if few else None,
+                                     few)
     _lib.check(lib.dfmi_switch_glu(
         x2.data_ptr(), _runtime.dtype_code(x.dtype), T, ids.data_ptr(), ids.element_size(), k,
         wg.data_ptr(), sg.data_ptr(), bg.data_ptr(), wu.data_ptr(), su.data_ptr(), bu.data_ptr(),
-        wd.data_ptr(), sd.data_ptr(), bd.data_ptr(), tg, td, h.data_ptr(), y.data_ptr(), D, I, E,
+        wd.data_ptr(), sd.data_ptr(), bd.data_ptr(), _ptr(glu), _ptr(dn), h.data_ptr(), y.data_ptr(), D, I, E,
         int(group_size), int(bits), scratch.data_ptr(), scratch.numel(), gws, gws_bytes,
         _runtime.stream_ptr(dev)),
         "dfmi_switch_glu")

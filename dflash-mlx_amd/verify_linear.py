@@ -31,8 +31,8 @@ from .verify_qmm import (
     _m4_ksplit_np_shape,
     _resolve_m16_ktmpl_variant,
     current_stream,
-    qmm_fused_launch,
     qmm_launch,
+    qmm_multi_launch,
     quantized_matmul,
     verify_matmul,
 )
@@ -209,19 +209,12 @@ class _VerifyState:
         self.gidx = 0
         self.vers = None
 
-    def current_table(self, obj):
-        """The pair table, if the module's tensors are still the ones it was
-        built from, unchanged (None: not, or a graph is being captured before
-        it exists)."""
-        if not self.pairs_ok or obj.weight is not self.w or obj.scales is not self.s or \
-                obj.biases is not self.b:
-            return None
-        if self.pairs is None and torch.cuda.is_current_stream_capturing():
-            return None
-        t = self.pair_table()
-        return t if self.table_current() else None
+    def holds(self, obj) -> bool:
+        """The module's tensors are the ones of this state."""
+        return obj.weight is self.w and obj.scales is self.s and obj.biases is self.b
 
-    def table_current(self) -> bool:
+    def unchanged(self) -> bool:
+        """Scales and biases are as they were when the pair table was built."""
         return self.vers is not None and self.vers == _runtime.versions((self.s, self.b))
 
     def pair_table(self):
@@ -319,16 +312,10 @@ def _build_dispatch(obj: VerifyQuantizedLinear, *, enable_qmm: Optional[bool] = 
                 if len(shp) != 2:
                     y = y.view(*shp[:-1], N)
             elif (x.dtype == sdt and x.is_cuda and m > 32 and kx == K and mode == "affine"
-                  and (t := state.current_table(obj)) is not None):
-                # many rows: the stock route, with the table the module holds,
-                # or as one launch with its siblings
-                grp = state.group
-                y = (grp.product(state.gidx, x, m, current_stream(x.get_device()))
-                     if grp is not None and not x.is_inference() else None)
-                if y is None:
-                    y = qmm_launch(_runtime.aligned_contiguous(x.reshape(m, kx)), state.w, state.s,
-                                   state.b, N, gs, bits, pairs=t, pair_stride=state.stride)
-                y = y.view(*shp[:-1], N)
+                  and state.group is not None and state.holds(obj) and not x.is_inference()):
+                # many rows: the stock route, or one launch with the siblings
+                y = state.group.product(state.gidx, x, m, current_stream(x.get_device()))
+                y = _stock(x) if y is None else y.view(*shp[:-1], N)
             else:
                 y = _stock(x)
             return y + bias if bias is not None else y
@@ -408,8 +395,9 @@ class SiblingGroup:
     The first member called with an input computes the product of every
     active member in one shared-activation launch (``dfmi_qmm_run`` on the
     group's prepared launch, the members' pair tables side by side in one
-    combined table; beyond 32 rows ``dfmi_qmm_affine_multi_fused`` where every
-    member is active and has such a table); each other member returns
+    combined table; beyond 32 rows, where every member is active and its scales
+    are as they were at install, one ``qmm_multi_launch`` that builds the tables
+    it reads from the scales); each other member returns
     its own product when it is called with the same tensor object, unchanged
     (same ``_version``) and on the same stream -- in the model's call order,
     with no change to the model code.  The group holds that input until every
@@ -488,11 +476,11 @@ class SiblingGroup:
         self.reset()
 
     def _takes_many(self, active) -> bool:
-        """More than 32 rows run as one launch: every member active, their
-        tables side by side and built from the scales as they are."""
+        """More than 32 rows run as one launch: two or three members, every one
+        active, their scales as installed (those that count versions)."""
         return (self.fused is not None and 2 <= len(self.states) <= 3
                 and len(active) == len(self.states)
-                and all(q.table_current() and not q.w.is_inference() for q in self.states))
+                and all(q.unchanged() and not q.w.is_inference() for q in self.states))
 
     def product(self, idx: int, x: torch.Tensor, m: int, st: int) -> Optional[torch.Tensor]:
         """Member idx's [m, N] product of x, or None when idx is not in the
@@ -509,7 +497,8 @@ class SiblingGroup:
                     self._miss[idx] = 0
                     if not ys:
                         self._pending = None  # every output taken: let the input go
-                    if vers is None or vers[idx] == self.states[idx].w._version:
+                    q = self.states[idx]
+                    if vers is None or vers[idx] == _runtime.versions((q.w, q.s, q.b)):
                         return y
         active = self.active
         if idx not in active:
@@ -534,9 +523,9 @@ class SiblingGroup:
         vers = None
         if many:
             first = self.states[0]
-            vers = [q.w._version for q in self.states]
-            qmm_fused_launch(x2, [(q.w, q.s, q.b) for q in self.states], self.fused, first.gs,
-                             first.bits, outs)
+            vers = [_runtime.versions((q.w, q.s, q.b)) for q in self.states]
+            qmm_multi_launch(x2, [(q.w, q.s, q.b) for q in self.states], first.gs, first.bits,
+                             outs=outs)
         else:
             rec = self._recs.get((m, st, x.dtype, active)) or self._record(m, st, x, active)
             rec.run(x2, outs, st)

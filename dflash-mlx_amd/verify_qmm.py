@@ -109,13 +109,10 @@ def _kparts_tuning():
 def _pairs_of(M: int, K: int, N: int, group_size: int, bits: int, scales, biases,
               pairs) -> Optional[torch.Tensor]:
     """The pair table a launch passes: the given one, else the functional
-    cache's for shapes whose plan can use it (None: none)."""
-    if pairs is None:
-        if _runtime.many_rows(M):
-            if K % group_size or K // group_size * N * 4 > 0xFFFFFFFF:
-                return None
-        elif not _runtime.pair_shape(M, K, N, group_size, bits):
-            return None
+    cache's for shapes whose streaming plan can use it (None: none; beyond 32
+    rows the library builds the table from the scales as they are, in the
+    call's scratch)."""
+    if pairs is None and _runtime.pair_shape(M, K, N, group_size, bits):
         pairs = _runtime.PAIRS.get(scales, biases)
     return pairs
 
@@ -130,12 +127,12 @@ def _pairs_ptr(M: int, K: int, N: int, group_size: int, bits: int, scales, biase
 def qmm_launch(x2: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
                N: int, group_size: int, bits: int, tuning=None,
                out: Optional[torch.Tensor] = None,
-               pairs: Optional[torch.Tensor] = None, pair_stride: int = 0) -> torch.Tensor:
+               pairs: Optional[torch.Tensor] = None) -> torch.Tensor:
     """One ``dfmi_qmm_affine_pairs`` launch on the current stream:
     ``[M, K] -> [M, N]``.  ``pairs`` is the layer's pair table
-    (``_runtime.build_sb_pairs``), or its column slice of a wider table of
-    ``pair_stride`` columns; when None, the one cached for ``scales`` is used
-    (built on first use).  The result does not depend on it."""
+    (``_runtime.build_sb_pairs``); when None, the one cached for ``scales`` is
+    used (built on first use; at most 32 rows).  The result does not depend on
+    it."""
     lib = _lib.load()
     M, K = x2.shape
     dev = x2.device
@@ -143,13 +140,6 @@ def qmm_launch(x2: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: 
     tptr = ctypes.byref(tuning) if tuning is not None else None
     need = int(lib.dfmi_qmm_workspace_bytes_ex(M, K, N, int(group_size), int(bits), tptr))
     ws, ws_bytes, _scratch = _runtime.launch_space(M, dev, need)
-    if pair_stride and tuning is None:
-        status = lib.dfmi_qmm_affine_pairs_strided(
-            x2.data_ptr(), _runtime.dtype_code(x2.dtype), w.data_ptr(), scales.data_ptr(),
-            biases.data_ptr(), pairs.data_ptr(), int(pair_stride), y.data_ptr(), M, K, N,
-            int(group_size), int(bits), ws, ws_bytes, _runtime.stream_ptr(dev))
-        _lib.check(status, "dfmi_qmm_affine_pairs_strided")
-        return y
     tp = _pairs_ptr(M, K, N, group_size, bits, scales, biases, pairs)
     status = lib.dfmi_qmm_affine_pairs(
         x2.data_ptr(), _runtime.dtype_code(x2.dtype), w.data_ptr(), scales.data_ptr(),
@@ -188,9 +178,8 @@ def qmm_multi_launch(x2: torch.Tensor, mats, group_size: int, bits: int,
     ws, ws_bytes, _scratch = _runtime.launch_space(M, dev, need)
     # two or three matrices with tables: the tables side by side, so that the
     # fused kernel starts its first loads without reading a segment table
-    # (many rows: the matrix-core kernel takes them apart as well)
     fused = (_runtime.FUSED_PAIRS.get(tables)
-             if 2 <= n <= 3 and not _runtime.many_rows(M) and all(t is not None for t in tables) else None)
+             if 2 <= n <= 3 and all(t is not None for t in tables) else None)
     if fused is not None:
         status = lib.dfmi_qmm_affine_multi_fused(
             x2.data_ptr(), _runtime.dtype_code(x2.dtype), segs, n, fused.data_ptr(), M, K,
@@ -202,29 +191,6 @@ def qmm_multi_launch(x2: torch.Tensor, mats, group_size: int, bits: int,
                                        _runtime.stream_ptr(dev))
     _lib.check(status, "dfmi_qmm_affine_multi")
     return ys
-
-
-def qmm_fused_launch(x2: torch.Tensor, mats, fused: torch.Tensor, group_size: int, bits: int,
-                     outs) -> None:
-    """One ``dfmi_qmm_affine_multi_fused`` launch of the sibling matrices
-    ``mats = [(w, scales, biases), ...]`` (2 or 3) whose pair tables stand side
-    by side in ``fused``, into ``outs``."""
-    lib = _lib.load()
-    M, K = int(x2.shape[0]), int(x2.shape[1])
-    dev = x2.device
-    n = len(mats)
-    segs = (_lib.QmmSegment * n)()
-    ns = (ctypes.c_int64 * n)()
-    for i, ((w, sc, bi), y) in enumerate(zip(mats, outs)):
-        segs[i].w_q, segs[i].scales, segs[i].biases = w.data_ptr(), sc.data_ptr(), bi.data_ptr()
-        segs[i].y, segs[i].N = y.data_ptr(), int(w.shape[0])
-        ns[i] = int(w.shape[0])
-    need = int(lib.dfmi_qmm_multi_workspace_bytes(M, K, ns, n, int(group_size), int(bits)))
-    ws, ws_bytes, _scratch = _runtime.launch_space(M, dev, need)
-    status = lib.dfmi_qmm_affine_multi_fused(
-        x2.data_ptr(), _runtime.dtype_code(x2.dtype), segs, n, fused.data_ptr(), M, K,
-        int(group_size), int(bits), ws, ws_bytes, _runtime.stream_ptr(dev))
-    _lib.check(status, "dfmi_qmm_affine_multi_fused")
 
 
 _raw_stream = torch._C._cuda_getCurrentRawStream

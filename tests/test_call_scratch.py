@@ -1,8 +1,10 @@
 """Host side of the calls that enqueue several kernels and pass data between
 them through scratch (more than 32 rows, more than 256 routed pairs, the expert
-sort): two calls in flight on one stream share no byte of it.  CPU only: a
-stand-in library records the scratch each call brings and holds the first call
-inside the library until the second one has been there."""
+sort): two calls in flight on one stream share no byte of it, and none of them
+brings a table kept from an earlier call.  On the CPU a stand-in library
+records what each call brings and holds the first call inside the library
+until the second one has been there; on the GPU two threads call on one
+stream."""
 
 from __future__ import annotations
 
@@ -128,6 +130,51 @@ def _from_two_threads(calls, check):
     for t in threads:
         t.join()
     assert not errors, errors[0]
+
+
+def test_no_kept_tables(library, monkeypatch):
+    """More than 32 rows bring no pair table, more than 256 pairs one built in
+    the call; 32 rows and 256 pairs take the cached ones."""
+    kept = torch.zeros(1)
+    monkeypatch.setattr(_runtime.PAIRS, "get", lambda *a, **k: kept)
+    tables = []
+
+    class Lib(_Library):
+        def __getattr__(self, name):
+            def call(*args):
+                if name.endswith("bytes") or name.endswith("bytes_ex"):
+                    return 65536 + 4096
+                tables.append(name)
+                if name == "dfmi_qmm_affine_pairs":
+                    tables.append(args[5])
+                elif name == "dfmi_qmm_affine_multi":
+                    tables.extend(args[2][i].sb_pairs for i in range(args[3]))
+                elif name in ("dfmi_gather_qmm_affine_pairs", "dfmi_moe_pairs"):
+                    tables.append(args[6] if "gather" in name else args[8])
+                return _lib.DFMI_OK
+            return call
+
+    monkeypatch.setattr(_lib, "load", lambda: Lib("", ()))
+    monkeypatch.setattr(_runtime.FUSED_PAIRS, "get", lambda tables: None)
+    w = _weights(128, 512)
+    for M in (33, 32):
+        x = torch.zeros((M, 512), dtype=torch.bfloat16)
+        vq.quantized_matmul(x, *w)
+        vq.quantized_matmul_multi(x, [w, w])
+        t = kept.data_ptr() if M == 32 else None
+        assert [a or None for a in tables] == ["dfmi_qmm_affine_pairs", t, "dfmi_qmm_affine_multi",
+                                               t, t]
+        tables.clear()
+    e = _weights(128, 512, lead=(4,))
+    for P in (257, 256):
+        x = torch.zeros((P, 512), dtype=torch.bfloat16)
+        moe.gather_qmm(x, *e, torch.zeros(P, dtype=torch.int32))
+        if P == 257:
+            assert tables == ["dfmi_moe_pairs", tables[1], "dfmi_gather_qmm_affine_pairs",
+                              tables[1]] and tables[1] not in (None, kept.data_ptr())
+        else:
+            assert tables == ["dfmi_gather_qmm_affine_pairs", kept.data_ptr()]
+        tables.clear()
 
 
 @pytest.mark.gpu

@@ -146,8 +146,6 @@ def test_matrices_in_one_launch(dev, M, K, Ns, gs, bits, dtype):
     check([vq.quantized_matmul(x, *m, group_size=gs, bits=bits) for m in mats])
     fused = torch.cat([_runtime.build_sb_pairs(s, b) for _, s, b in mats], dim=1).contiguous()
     outs = [torch.full_like(y, float("nan")) for y in one]
-    vq.qmm_fused_launch(x, mats, fused, gs, bits, outs)
-    assert all(torch.equal(a, b) for a, b in zip(one, outs))
     segs = (_lib.QmmSegment * len(mats))()
     for g, (w, s, b), y in zip(segs, mats, outs):
         g.w_q, g.scales, g.biases = w.data_ptr(), s.data_ptr(), b.data_ptr()
@@ -165,6 +163,12 @@ def test_matrices_in_one_launch(dev, M, K, Ns, gs, bits, dtype):
     rc = _lib.load().dfmi_qmm_affine_multi(  # tables into the workspace, for the call
         x.data_ptr(), _runtime.dtype_code(x.dtype), segs, len(mats), M, K, gs, bits, ws, ws_bytes,
         _runtime.stream_ptr(x.device))
+    assert rc == _lib.DFMI_OK and all(torch.equal(a, b) for a, b in zip(one, outs))
+    for y in outs:
+        y.fill_(float("nan"))
+    rc = _lib.load().dfmi_qmm_affine_multi_fused(
+        x.data_ptr(), _runtime.dtype_code(x.dtype), segs, len(mats), fused.data_ptr(), M, K, gs,
+        bits, ws, ws_bytes, _runtime.stream_ptr(x.device))
     assert rc == _lib.DFMI_OK and all(torch.equal(a, b) for a, b in zip(one, outs))
 
 
@@ -253,3 +257,61 @@ def test_module_many_rows(dev):
         for m in (gate, up, down):
             want1 = vq.quantized_matmul(x, m.weight, m.scales, m.biases, group_size=gs, bits=4)
             assert torch.equal(m(x), want1)
+
+
+@pytest.mark.parametrize("route", ["operator", "siblings", "module", "group"])
+def test_scales_are_read_at_each_call(dev, route):
+    """Beyond 32 rows the product is of the scales as they are: after an
+    update that counts no version, and in a graph replayed after one, also
+    when eager calls and other allocations came between."""
+    import torch
+    from torch import nn
+
+    from dflash_mlx_amd import verify_linear as vl, verify_qmm as vq
+
+    M, K, Ns, gs = 45, 2048, (384, 256), 64
+    mats, x = [], None
+    for i, N in enumerate(Ns):
+        _, (xi, w, s, b) = _case(dev, M, K, N, gs, 4, "bf16", seed=70 + i)
+        x = xi if x is None else x
+        mats.append((w, s, b))
+    root = nn.Module()
+    root.mlp = nn.Module()
+    for name, (w, s, b) in zip(("gate_proj", "up_proj"), mats):
+        setattr(root.mlp, name, vl.QuantizedLinear(w, s, b, group_size=gs, bits=4))
+    vl.install_verify_linears(root, enable_qmm=True, fuse_siblings=route == "group")
+
+    def run(a):
+        if route == "operator":
+            return [vq.quantized_matmul(a, *m, group_size=gs, bits=4) for m in mats]
+        if route == "siblings":
+            return vq.quantized_matmul_multi(a, mats, group_size=gs, bits=4)
+        return [root.mlp.gate_proj(a), root.mlp.up_proj(a)]
+
+    def want():  # the same values in tensors the library has not seen
+        fresh = [tuple(t.clone() for t in m) for m in mats]
+        if route in ("siblings", "group"):
+            return vq.quantized_matmul_multi(x.clone(), fresh, group_size=gs, bits=4)
+        return [vq.quantized_matmul(x, *m, group_size=gs, bits=4) for m in fresh]
+
+    def same(got, ref):
+        torch.cuda.synchronize()
+        assert all(torch.equal(g, r) for g, r in zip(got, ref))
+
+    same(run(x.clone()), want())
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        ys = run(x)
+    for step in range(3):
+        for _, s, b in mats:
+            for t in (s, b):
+                t.data.copy_(torch.roll(t, 1 + step, 0))  # counts no version of s, b
+        ref = want()
+        graph.replay()
+        same(ys, ref)
+        same(run(x.clone()), ref)
+        junk = [torch.full((m[1].numel(),), float("nan"), device=dev) for m in mats * 8]
+        graph.replay()
+        same(ys, ref)
+        del junk

@@ -151,3 +151,40 @@ def test_switch_glu_captured(dev):
             hr, yr = _reference(torch, x, inds, gate, up, down, gs)
             _close(torch, h, hr)
             _close(torch, y, yr)
+
+
+def test_scales_are_read_at_each_call(dev):
+    """Beyond 256 pairs the results are of the scales as they are: after an
+    update that counts no version, and in a graph replayed after one."""
+    import torch
+
+    from dflash_mlx_amd import moe
+
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(12)
+    E, D, I, gs = 16, 256, 128, 64
+    gate, up = (_experts(torch, gen, E, I, D, gs, torch.bfloat16, dev) for _ in range(2))
+    down = _experts(torch, gen, E, D, I, gs, torch.bfloat16, dev)
+    x = torch.randn((50, D), generator=gen, device=dev).to(torch.bfloat16)
+    inds = torch.randint(0, E, (50, 8), generator=gen, device=dev)
+    rhs, lhs = inds.reshape(-1), torch.arange(400, device=dev) // 8
+
+    def run():
+        h = moe.gather_swiglu(x, gate, up, rhs, lhs_indices=lhs, group_size=gs)
+        return (*moe.switch_glu(x, inds, gate, up, down, group_size=gs), h,
+                moe.gather_qmm(h, *down, rhs, group_size=gs))
+
+    run()
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        ys = run()
+    for step in range(3):
+        for t in (*gate[1:], *up[1:], *down[1:]):
+            t.data.copy_(torch.roll(t, 1 + step, 0))
+        hr, yr = _reference(torch, x, inds, gate, up, down, gs)
+        graph.replay()
+        torch.cuda.synchronize()
+        for got in (ys, run()):
+            for g, r in zip(got, (hr, yr, hr, yr)):
+                _close(torch, g, r)

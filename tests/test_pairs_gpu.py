@@ -94,6 +94,37 @@ def test_sb_pairs_layout(dev, N, G, dtype):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("E,N,G,two", [
+    (1, 256, 8, 0), (1, 260, 16, 0), (1, 1028, 24, 0), (1, 66, 32, 0), (1, 4, 272, 0),
+    (3, 96, 8, 1), (2, 32, 16, 1), (2, 160, 40, 1), (3, 64, 33, 1),
+])
+def test_pair_table_tiles(dev, E, N, G, two, off):
+    """Each tile of the table kernel (1, 2 and 4 lanes along the groups) at
+    its edges, one set and two, also from arrays off a 16-byte boundary: the
+    bits of the scales and biases."""
+    import torch
+
+    from dflash_mlx_amd import _runtime
+
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(N + G)
+    sets = []
+    for _ in range(4 if two else 2):
+        flat = torch.randint(-2 ** 15, 2 ** 15, (E * N * G + off,), generator=gen, device=dev,
+                             dtype=torch.int16)
+        sets.append(flat[off:].view(torch.bfloat16).reshape(E, N, G))
+    bits = [a.view(torch.int16).to(torch.int32) & 0xFFFF for a in sets]
+    want = bits[0] | bits[1] << 16
+    if two:
+        up = bits[2] | bits[3] << 16
+        want = torch.stack([want.reshape(E, N // 32, 32, G), up.reshape(E, N // 32, 32, G)], 2)
+        want = want.reshape(E, 2 * N, G)
+    got = (_runtime.build_moe_pairs(*sets) if E > 1 or two
+           else _runtime.build_sb_pairs(sets[0][0], sets[1][0])[None])
+    assert torch.equal(got, want.transpose(1, 2))
+
+
 @pytest.mark.parametrize("M,K,N,gs", [
     (16, 4096, 4096, 64),        # 64 blocks: 4 splits, one workgroup per CU
     (16, 17408, 5120, 64),       # 68 steps: 6 splits, two per CU
