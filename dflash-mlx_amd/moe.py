@@ -218,6 +218,9 @@ def _switch_glu(x, inds, gate: Triple, up: Triple, down: Triple, group_size: int
     The pair order lies in scratch of the call's own."""
     _runtime.require_device(x, "x")
     dev = x.device
+    for t in (inds, *gate, *up, *down):
+        if t.device != dev:
+            raise ValueError(f"x is on {dev}, expert ids or weights on {t.device}")
     T, k = int(inds.shape[0]), int(inds.shape[1])
     D = int(x.shape[-1])
     x2 = _runtime.aligned_contiguous(x.reshape(-1, D))

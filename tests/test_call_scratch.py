@@ -132,6 +132,20 @@ def _from_two_threads(calls, check):
     assert not errors, errors[0]
 
 
+def test_expert_tensors_on_another_device(library):
+    """switch_glu refuses expert ids or weights that are not where x is, before
+    anything reaches the library."""
+    gate, down = _weights(128, 256, lead=(4,)), _weights(256, 128, lead=(4,))
+    x, ids = torch.zeros((16, 256), dtype=torch.bfloat16), torch.zeros((16, 8), dtype=torch.int32)
+    for at in range(10):
+        lib = library("dfmi_switch_glu", ())
+        lib.second.set()
+        ts = [t.to("meta") if i == at else t for i, t in enumerate((ids, *gate, *gate, *down))]
+        with pytest.raises(ValueError, match="on meta"):
+            moe._switch_glu(x, ts[0], ts[1:4], ts[4:7], ts[7:10], 64, 4)
+        assert not lib.seen
+
+
 def test_no_kept_tables(library, monkeypatch):
     """More than 32 rows bring no pair table, more than 256 pairs one built in
     the call; 32 rows and 256 pairs take the cached ones."""

@@ -188,3 +188,22 @@ def test_scales_are_read_at_each_call(dev):
         for got in (ys, run()):
             for g, r in zip(got, (hr, yr, hr, yr)):
                 _close(torch, g, r)
+
+
+def test_expert_weights_off_the_gpu_are_refused(dev):
+    import torch
+
+    from dflash_mlx_amd import moe
+
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(1)
+    gate = _experts(torch, gen, 4, 128, 256, 64, torch.bfloat16, dev)
+    down = _experts(torch, gen, 4, 256, 128, 64, torch.bfloat16, dev)
+    x = torch.randn((3, 256), generator=gen, device=dev).to(torch.bfloat16)
+    inds = torch.zeros((3, 2), dtype=torch.int32, device=dev)
+    for i in range(3):
+        host = tuple(t.cpu() if j == i else t for j, t in enumerate(down))
+        with pytest.raises(ValueError):
+            moe.switch_glu(x, inds, gate, gate, host)
+    with pytest.raises(ValueError):
+        moe.switch_glu(x, inds.cpu(), gate, gate, down)
