@@ -69,10 +69,17 @@ static size_t table_bytes(int64_t K, int64_t N, int gs) {
   return round_up((size_t)(K / gs) * (size_t)N * 4u, 256);
 }
 
+// Bytes of a pair table a DMA may step through: lanes without a row read at
+// kNoRow plus the step's offset, which stays past the table's end and below
+// 2^32 only if the table is below 2^31.
+static bool table_fits(int64_t K, int64_t cols, int gs) {
+  return (K / gs) * cols * 4 < (1ll << 31);
+}
+
 // More rows than the streaming kernels take; 32-bit byte offsets within a
 // tile's rows and the pair table.
 bool gemm_shape(int64_t M, int64_t K, int64_t N, int gs) {
-  return M > 32 && K < (1ll << 23) && (K / gs) * N * 4 <= 0xFFFFFFFFll &&
+  return M > 32 && K < (1ll << 23) && table_fits(K, N, gs) &&
          ((M + 31) / 32) * ((N + 127) / 128) < (1ll << 24);
 }
 
@@ -125,6 +132,7 @@ static size_t gemm_space(void* workspace, size_t bytes, char*& ws) {
 int gemm_launch(const void* x, int x_dtype, const dfmi_qmm_segment* segs, int nseg,
                 const uint32_t* fused, int64_t pair_stride, int64_t M, int64_t K, int gs,
                 int bits, void* workspace, size_t workspace_bytes, hipStream_t st) {
+  if (pair_stride && !table_fits(K, pair_stride, gs)) return kGemmNotTaken;
   // (tables, product and split sum pass data through the workspace)
   std::lock_guard<std::mutex> order(launch_order());
   char* ws;

@@ -235,3 +235,15 @@ def test_streaming_split_plans(lib):
 def _lib_tuning(path, tiles, waves, splits, rows=0):
     from dflash_mlx_amd import _lib
     return _lib.QmmTuning(path, tiles, waves, splits, rows)
+
+
+def test_pair_tables_of_two_gigabytes(lib):
+    """The matrix-core kernel's DMA takes "no row" offsets past tables below
+    2^31 bytes: larger ones go to the general kernel, without a workspace."""
+    for N, name in (((1 << 19) - 4, b"qmm_gemm_kernel"), (1 << 19, b"qmm_dense_kernel"),
+                    ((1 << 20) - 4, b"qmm_dense_kernel")):
+        assert lib.dfmi_qmm_kernel_name(64, 32768, N, 32, 4, None) == name
+        assert (lib.dfmi_qmm_workspace_bytes(64, 32768, N, 32, 4) > 0) == (b"gemm" in name)
+    ns = (ctypes.c_int64 * 2)(1 << 18, 1 << 18)  # side by side
+    one = lib.dfmi_qmm_workspace_bytes(64, 32768, 1 << 18, 32, 4)
+    assert lib.dfmi_qmm_multi_workspace_bytes(64, 32768, ns, 2, 32, 4) == one
