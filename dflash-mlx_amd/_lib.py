@@ -74,6 +74,7 @@ _SIGNATURES = {
     "dfmi_qmm_affine_pairs_strided": (_int, [_c_void_p, _int, _c_void_p, _c_void_p, _c_void_p,
                                              _c_void_p, _i64, _c_void_p, _i64, _i64, _i64, _int,
                                              _int, _c_void_p, _size, _c_void_p]),
+    "dfmi_capture_id": (ctypes.c_ulonglong, [_c_void_p]),
     "dfmi_sb_pairs": (_int, [_c_void_p, _c_void_p, _int, _i64, _i64, _c_void_p, _c_void_p]),
     "dfmi_qmm_plan": (_int, [_i64, _i64, ctypes.POINTER(ctypes.c_int64), _int, _int, _int,
                              ctypes.POINTER(QmmTuning), ctypes.POINTER(QmmPlanInfo)]),

@@ -42,6 +42,13 @@ def stream_ptr(device: torch.device) -> int:
     return _raw_stream(torch.cuda.current_device() if index is None else index)
 
 
+def capture_key(stream: int) -> int:
+    """0 for the current stream running, or which graph capture it is in."""
+    if not torch.cuda.is_current_stream_capturing():
+        return 0
+    return 1 + int(_lib.load().dfmi_capture_id(stream))
+
+
 def aligned_contiguous(t: torch.Tensor) -> torch.Tensor:
     """Contiguous tensor whose data pointer is 16-byte aligned (copy if needed)."""
     t = t.contiguous()

@@ -28,3 +28,12 @@ std::mutex& launch_order() {
 extern "C" const char* dfmi_version(void) { return "dfmi 0.1.0 gfx950"; }
 
 extern "C" const char* dfmi_last_error(void) { return dfmi::g_error.c_str(); }
+
+extern "C" unsigned long long dfmi_capture_id(void* stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (hipStreamGetCaptureInfo(static_cast<hipStream_t>(stream), &status, &id) != hipSuccess ||
+      status != hipStreamCaptureStatusActive)
+    return 0;
+  return id;
+}

@@ -399,7 +399,8 @@ class SiblingGroup:
     are as they were at install, one ``qmm_multi_launch`` that builds the tables
     it reads from the scales); each other member returns
     its own product when it is called with the same tensor object, unchanged
-    (same ``_version``) and on the same stream -- in the model's call order,
+    (same ``_version``) and on the same stream, both calls eager or in the same
+    graph capture -- in the model's call order,
     with no change to the model code.  The group holds that input until every
     active member has taken its output, so its storage cannot be reused for
     another tensor meanwhile.  A member called with any other input launches
@@ -486,8 +487,9 @@ class SiblingGroup:
         """Member idx's [m, N] product of x, or None when idx is not in the
         shared launch (the member then launches alone)."""
         many = m > 32
-        # (a captured launch computes nothing until its graph is replayed)
-        where = (st, torch.cuda.is_current_stream_capturing()) if many else st
+        # (a captured launch computes nothing until its own graph is replayed,
+        # and a replay nothing that was launched before)
+        where = (st, _runtime.capture_key(st))
         pending = self._pending
         if pending is not None:
             held, ver, there, ys, vers = pending

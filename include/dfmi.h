@@ -49,6 +49,8 @@ extern "C" {
 /* Library version string and the message of the last failed call on this thread. */
 const char *dfmi_version(void);
 const char *dfmi_last_error(void);
+/* Id of the graph capture a stream is in (hipStreamGetCaptureInfo), or 0. */
+unsigned long long dfmi_capture_id(void *stream);
 
 /* Optional launch-shape override for the affine qmm (tuning sweeps).  Zero
  * fields mean "automatic".
