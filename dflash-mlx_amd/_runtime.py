@@ -203,27 +203,25 @@ def versions(tensors) -> Optional[tuple]:
 
 
 class _Built:
-    """A table and when it is there: a call on another stream than the one
-    that builds it waits for it on the device.  (During capture nothing is
-    waited for: a capture begins behind a synchronised device.)"""
+    """A table and when it is there: the first call on another stream than the
+    one that builds it waits for it on the device (no event is queried: that
+    would break a capture another thread has running).  During capture
+    nothing is waited for: a capture begins behind a synchronised device."""
 
-    __slots__ = ("table", "device", "stream", "event")
+    __slots__ = ("table", "device", "event", "streams")
 
     def __init__(self, table: torch.Tensor):
         self.table = table
         self.device = table.get_device()
-        self.stream = _raw_stream(self.device)
         self.event = torch.cuda.Event()
         self.event.record(torch.cuda.current_stream(self.device))
+        self.streams = {_raw_stream(self.device)}  # those it is there for
 
     def get(self) -> torch.Tensor:
-        event = self.event
-        if (event is not None and _raw_stream(self.device) != self.stream
-                and not torch.cuda.is_current_stream_capturing()):
-            if event.query():
-                self.event = None
-            else:
-                torch.cuda.current_stream(self.device).wait_event(event)
+        st = _raw_stream(self.device)
+        if st not in self.streams and not torch.cuda.is_current_stream_capturing():
+            torch.cuda.current_stream(self.device).wait_event(self.event)
+            self.streams.add(st)
         return self.table
 
 

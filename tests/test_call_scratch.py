@@ -132,6 +132,36 @@ def _from_two_threads(calls, check):
     assert not errors, errors[0]
 
 
+def test_tables_are_waited_for_once_per_stream(monkeypatch):
+    """A table is waited for on the device by the first call on each stream but
+    the one that built it, never while capturing, and its event not queried."""
+    waits, at = [], {"stream": 1, "capturing": False}
+
+    class Event:
+        def record(self, stream):
+            waits.append(("record", stream))
+
+        def query(self):
+            raise AssertionError("queried")
+
+    class Stream:
+        def wait_event(self, event):
+            waits.append(at["stream"])
+
+    monkeypatch.setattr(torch.cuda, "Event", Event)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda d: Stream())
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: at["capturing"])
+    monkeypatch.setattr(_runtime, "_raw_stream", lambda d: at["stream"])
+    table = torch.zeros(4)
+    built = _runtime._Built(table)
+    waits.clear()
+    for stream, capturing in ((1, False), (2, False), (2, False), (3, True), (3, False), (1, False),
+                              (2, False), (3, False)):
+        at.update(stream=stream, capturing=capturing)
+        assert built.get() is table
+    assert waits == [2, 3]
+
+
 def test_expert_tensors_on_another_device(library):
     """switch_glu refuses expert ids or weights that are not where x is, before
     anything reaches the library."""
