@@ -195,7 +195,7 @@ class _VerifyState:
     and the sibling group it belongs to."""
 
     __slots__ = ("w", "s", "b", "N", "K", "gs", "bits", "pairs", "pairs_ok", "stride", "recs",
-                 "group", "gidx", "vers")
+                 "group", "gidx", "vers", "built")
 
     def __init__(self, w, s, b, N, K, gs, bits):
         self.w, self.s, self.b = w, s, b
@@ -208,6 +208,7 @@ class _VerifyState:
         self.group = None
         self.gidx = 0
         self.vers = None
+        self.built: Optional[_runtime._Built] = None  # of the table pairs is (a slice of)
 
     def holds(self, obj) -> bool:
         """The module's tensors are the ones of this state."""
@@ -227,6 +228,7 @@ class _VerifyState:
                 _warn_capture_without_table()
                 return None
             self.pairs = _runtime.build_sb_pairs(self.s, self.b)
+            self.built = _runtime._Built(self.pairs)
             self.vers = _runtime.versions((self.s, self.b))
         return self.pairs
 
@@ -236,6 +238,8 @@ class _VerifyState:
         rec = self.recs.get(key)
         if rec is None:
             t = self.pair_table() if m <= 32 else None
+            if t is not None:
+                self.built.get()  # (there before this stream's first launch)
             rec = LaunchRecord(m, self.K, x.dtype, x.device, [(self.w, self.s, self.b, t)],
                                self.gs, self.bits, sb_stride=self.stride if t is not None else 0)
             if t is not None or not self.pairs_ok or m > 32:
@@ -439,6 +443,9 @@ class SiblingGroup:
             sts = [self.states[j] for j in active]
             first = sts[0]
             tabs = [st_.pair_table() for st_ in sts]
+            for q in sts:
+                if q.built is not None:
+                    q.built.get()
             # the combined table serves the launch of every member (the
             # fused kernel: two or three matrices of fewer than 2^16 rows);
             # otherwise each matrix reads its column slice of it
@@ -563,12 +570,15 @@ def _group_siblings(model: nn.Module) -> int:
             if all(t is not None for t in tabs) and all(q.N % 4 == 0 for q in states):
                 # (a member regrouped contributes its column slice of its old
                 # group's table)
+                for q in states:
+                    q.built.get()
                 fused = torch.cat(tabs, dim=1).contiguous()
                 stride = int(fused.shape[1])
+                built = _runtime._Built(fused)
                 c = 0
                 for q in states:  # the members' own tables are released
                     q.pairs = fused[:, c:c + q.N]
-                    q.stride = stride
+                    q.stride, q.built = stride, built
                     q.recs = {}
                     c += q.N
             grp = SiblingGroup(states, fused, stride)

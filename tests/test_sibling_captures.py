@@ -1,6 +1,7 @@
-"""Pending outputs of a sibling group and graph captures: a member takes what
-its group's launch computed only where that launch runs in the same place --
-both calls eager, or both in one capture -- at every row count."""
+"""Verify modules over streams and graph captures.  A member of a sibling group
+takes what its group's launch computed only where that launch runs in the same
+place -- both calls eager, or both in one capture -- at every row count; and a
+launch on another stream than the install's waits for the tables."""
 
 from __future__ import annotations
 
@@ -43,6 +44,69 @@ def test_outputs_stay_with_their_launch(monkeypatch, M):
         want = min(step + 1, 4)  # the last one is the eager launch before it
         assert len(launches) == want and torch.all(y == want)
     assert launches == [0, 7, 9, 0]
+
+
+def test_each_launch_prepared_waits_for_its_table(monkeypatch):
+    monkeypatch.setattr(vl, "LaunchRecord", lambda *a, **k: object())
+    gets = []
+
+    class Built:
+        def __init__(self, name):
+            self.name = name
+
+        def get(self):
+            gets.append(self.name)
+
+    bf = torch.bfloat16
+    states = []
+    for name in "ab":
+        w, s = torch.zeros((64, 32), dtype=torch.int32), torch.zeros((64, 4), dtype=bf)
+        q = vl._VerifyState(w, s, s, 64, 256, 64, 4)
+        q.pairs, q.built = torch.zeros(1), Built(name)
+        states.append(q)
+    x = torch.zeros((16, 256), dtype=bf)
+    for st in (5, 5, 6):
+        states[0].record(16, st, x)
+    assert gets == ["a", "a"]
+    gets.clear()
+    grp = vl.SiblingGroup(states, torch.zeros(1), 128)
+    for st in (5, 5, 6):
+        grp._record(16, st, x, (0, 1))
+    assert gets == ["a", "b"] * 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [16, 40])
+@pytest.mark.parametrize("fuse", [False, True])
+def test_call_on_another_stream_right_after_install(dev, M, fuse):
+    """Installed behind a long-running kernel of one stream, called on another
+    at once: the result of the finished tables."""
+    from torch import nn
+
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(M)
+    K, N, gs = 1024, 512, 64
+    x = torch.randn((M, K), generator=gen, device=dev).to(torch.bfloat16)
+    got, streams = {}, [torch.cuda.Stream(), torch.cuda.Stream()]
+    mats = [vl.QuantizedLinear.from_linear(nn.Linear(K, N, bias=False, device=dev), gs, 4,
+                                           torch.bfloat16) for _ in range(2)]
+    for late in (False, True):
+        root = nn.Module()
+        root.mlp = nn.Module()
+        for name, q in zip(("gate_proj", "up_proj"), mats):
+            setattr(root.mlp, name, vl.QuantizedLinear(
+                q.weight.clone(), q.scales.clone(), q.biases.clone(), group_size=gs, bits=4))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(streams[0]):
+            if late:
+                torch.cuda._sleep(100_000_000)
+            vl.install_verify_linears(root, enable_qmm=True, fuse_siblings=fuse)
+        if not late:
+            torch.cuda.synchronize()
+        with torch.cuda.stream(streams[1]):
+            got[late] = [root.mlp.gate_proj(x), root.mlp.up_proj(x)]
+        torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(got[False], got[True]))
 
 
 @pytest.mark.gpu
