@@ -78,6 +78,8 @@ _SIGNATURES = {
     "dfmi_sb_pairs": (_int, [_c_void_p, _c_void_p, _int, _i64, _i64, _c_void_p, _c_void_p]),
     "dfmi_qmm_plan": (_int, [_i64, _i64, ctypes.POINTER(ctypes.c_int64), _int, _int, _int,
                              ctypes.POINTER(QmmTuning), ctypes.POINTER(QmmPlanInfo)]),
+    "dfmi_qmm_gemm_plan": (_int, [_i64, _i64, ctypes.POINTER(ctypes.c_int64), _int, _int, _int]
+                           + [ctypes.POINTER(ctypes.c_int)] * 3),
     "dfmi_qmm_kernel_name": (ctypes.c_char_p, [_i64, _i64, _i64, _int, _int,
                                                ctypes.POINTER(QmmTuning)]),
     "dfmi_qmm_workspace_bytes_ex": (_size, [_i64, _i64, _i64, _int, _int,

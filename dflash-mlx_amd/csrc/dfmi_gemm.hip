@@ -94,6 +94,14 @@ size_t gemm_multi_workspace_bytes(int64_t M, int64_t K, const int64_t* Ns, int n
   return kGemmWsOffset + tables + gemm_plan(M, K, Ns, nseg, kGemmMaxPartials).partials;
 }
 
+void gemm_plan_query(int64_t M, int64_t K, const int64_t* Ns, int nseg, int* rows, int* cols,
+                     int* splits) {
+  const GemmPlan p = gemm_plan(M, K, Ns, nseg, kGemmMaxPartials);
+  *rows = kGemmCfgs[p.cfg].bm;
+  *cols = kGemmCfgs[p.cfg].bn;
+  *splits = p.kp;
+}
+
 // the planned launch of a whose matrices, table and rows are set
 static int gemm_run(GemmArgs& a, int x_dtype, int gs, int bits, char* ws, size_t left,
                     hipStream_t st) {

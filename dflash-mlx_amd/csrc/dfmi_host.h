@@ -49,6 +49,9 @@ constexpr int kGemmNotTaken = 1;
 bool gemm_shape(int64_t M, int64_t K, int64_t N, int gs);
 size_t gemm_workspace_bytes(int64_t M, int64_t K, int64_t N, int gs);
 size_t gemm_multi_workspace_bytes(int64_t M, int64_t K, const int64_t* Ns, int nseg, int gs);
+// tile and K splits of a launch with the whole workspace
+void gemm_plan_query(int64_t M, int64_t K, const int64_t* Ns, int nseg, int* rows, int* cols,
+                     int* splits);
 // fused: the matrices' tables side by side, or null (their own sb_pairs, rows
 // pair_stride apart if not 0).  More than one matrix: every N >= 1 and a
 // multiple of 4.

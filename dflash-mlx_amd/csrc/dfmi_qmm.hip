@@ -1060,6 +1060,24 @@ extern "C" int dfmi_qmm_plan(int64_t M, int64_t K, const int64_t* Ns, int nseg, 
   return DFMI_OK;
 }
 
+extern "C" int dfmi_qmm_gemm_plan(int64_t M, int64_t K, const int64_t* Ns, int nseg,
+                                  int group_size, int bits, int* tile_rows, int* tile_cols,
+                                  int* k_splits) {
+  if (!Ns || !tile_rows || !tile_cols || !k_splits || nseg < 1 || nseg > kMaxSeg) {
+    set_error("dfmi_qmm_gemm_plan: bad arguments");
+    return DFMI_EINVAL;
+  }
+  for (int i = 0; i < nseg; ++i) {
+    const int rc = validate_qmm(DFMI_BF16, M, K, Ns[i], group_size, bits);
+    if (rc != DFMI_OK) return rc;
+  }
+  *tile_rows = *tile_cols = *k_splits = 0;
+  if (nseg == 1 ? Ns[0] > 0 && use_gemm(M, K, Ns[0], group_size, nullptr)
+                : use_gemm_multi(M, K, Ns, nseg, group_size))
+    gemm_plan_query(M, K, Ns, nseg, tile_rows, tile_cols, k_splits);
+  return DFMI_OK;
+}
+
 extern "C" const char* dfmi_qmm_kernel_name(int64_t M, int64_t K, int64_t N, int group_size,
                                              int bits, const dfmi_qmm_tuning* tuning) {
   if (validate_qmm(DFMI_BF16, M, K, N, group_size, bits) != DFMI_OK || !valid_path(tuning))

@@ -198,9 +198,15 @@ typedef struct dfmi_qmm_plan_info {
 } dfmi_qmm_plan_info;
 int dfmi_qmm_plan(int64_t M, int64_t K, const int64_t *Ns, int nseg, int group_size, int bits,
                   const dfmi_qmm_tuning *tuning, dfmi_qmm_plan_info *out);
+/* Host-only plan query (no reference counterpart; for tests and profiles):
+ * tile and K splits of the matrix-core launch that one matrix (nseg 1), or
+ * two or three in one launch, make at M > 32 with the workspace; all 0 where
+ * another kernel, or a launch per matrix, runs. */
+int dfmi_qmm_gemm_plan(int64_t M, int64_t K, const int64_t *Ns, int nseg, int group_size, int bits,
+                       int *tile_rows, int *tile_cols, int *k_splits);
 /* Host-only plan query (no reference counterpart; for benchmarks and
  * profiles): name of the kernel dfmi_qmm_affine_ex would launch for this
- * shape, "qmm_stream_kernel", "qmm_dense_kernel" or
+ * shape, "qmm_stream_kernel", "qmm_dense_kernel", "qmm_gemm_kernel" or
  * (bits 8) "qmm8_stream_kernel" / "qmm8_kernel";
  * NULL if unsupported. */
 const char *dfmi_qmm_kernel_name(int64_t M, int64_t K, int64_t N, int group_size, int bits,

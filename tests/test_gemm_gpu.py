@@ -1,6 +1,8 @@
-"""GPU parity of ``qmm_gemm_kernel`` (more than 32 activation rows) against the
-CPU oracle at the edges of its tiles: 32-, 64- and 96-row blocks, 128- and
-256-column blocks, 128-k steps with a remainder, one and several K splits.
+"""GPU parity of ``qmm_gemm_kernel`` (more than 32 activation rows).  The small
+shapes, against the CPU oracle, are planned on its 32 x 128 tile;
+``test_every_tile`` takes each of the three tiles (32 x 128, 96 x 128, 64 x
+256), with one and several K splits, ragged rows, columns and K, against
+float64 sums, and checks which tile the plan took.
 
 Bound per output: one rounding to the output type (half an ulp: 2^-8 relative
 in bf16, 2^-11 in f16) plus the fp32 sum's worst case, K 2^-24 of the sum of
@@ -54,6 +56,78 @@ def test_tile_edges(dev, M, K, N, gs, bits, dtype):
     _check(from_dev(y, dtype), case, gs, bits, dtype)
     again = vq.quantized_matmul(x, w, s, b, group_size=gs, bits=bits)
     assert np.array_equal(from_dev(y, dtype), from_dev(again, dtype))
+
+
+def _plan(M, K, Ns, gs, bits):
+    from dflash_mlx_amd import _lib
+
+    ns, out = (ctypes.c_int64 * len(Ns))(*Ns), [ctypes.c_int() for _ in range(3)]
+    rc = _lib.load().dfmi_qmm_gemm_plan(M, K, ns, len(Ns), gs, bits,
+                                        *[ctypes.byref(v) for v in out])
+    assert rc == _lib.DFMI_OK
+    return tuple(v.value for v in out)
+
+
+def _random_weights(dev, gen, N, K, gs, bits, dt):
+    """Any codes; scales and biases of a weight of about 0.02."""
+    import torch
+
+    w = torch.randint(-2 ** 31, 2 ** 31 - 1, (N, K * bits // 32), generator=gen, device=dev,
+                      dtype=torch.int32)
+    s = (torch.rand((N, K // gs), generator=gen, device=dev) + 0.5) * (0.08 / 2 ** bits)
+    b = (torch.rand((N, K // gs), generator=gen, device=dev) - 1.5) * 0.04
+    return w, s.to(dt), b.to(dt)
+
+
+def _within(y, x, mat, gs, bits):
+    """y against float64 sums, by blocks of columns, to the bound above."""
+    import torch
+
+    w, s, b = mat
+    K, half = x.shape[1], 2.0 ** (-8 if y.dtype == torch.bfloat16 else -11)
+    shifts = torch.arange(32 // bits, device=w.device, dtype=torch.int32) * bits
+    for n in range(0, w.shape[0], 4096):
+        q = ((w[n:n + 4096, :, None] >> shifts) & (2 ** bits - 1)).reshape(-1, K).double()
+        sd, bd = (a[n:n + 4096].double().repeat_interleave(gs, 1) for a in (s, b))
+        ref = x.double() @ (q * sd + bd).T
+        mag = x.double().abs() @ (q * sd.abs() + bd.abs()).T
+        bound = half * ref.abs() + K * 2.0 ** -24 * mag
+        assert bool(((y[:, n:n + 4096].double() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("tile,split,M,K,Ns", [
+    ((32, 128), False, 65, 192, (129,)), ((32, 128), True, 65, 1088, (136,)),
+    ((32, 128), True, 500, 4160, (644, 4, 640)),
+    ((64, 256), False, 103, 64, (16388,)), ((64, 256), False, 1000, 192, (2504,)),
+    ((64, 256), False, 1000, 64, (2501,)), ((64, 256), True, 97, 2112, (8200,)),
+    ((64, 256), True, 500, 4160, (1284,)), ((64, 256), False, 1000, 192, (1028, 4, 1480)),
+    ((96, 128), False, 229, 64, (16388,)), ((96, 128), False, 500, 192, (8200,)),
+    ((96, 128), True, 77, 4160, (12296,)), ((96, 128), True, 65, 4160, (6148, 4, 6148)),
+])
+def test_every_tile(dev, tile, split, M, K, Ns, gs, bits, dtype):
+    import torch
+
+    from dflash_mlx_amd import verify_qmm as vq
+
+    # the same steps of 128 at every group size: K - 32, K and K + 64
+    K += {32: -32, 64: 0, 128: -K % 128}[gs]
+    rows, cols, kp = _plan(M, K, Ns, gs, bits)
+    assert (rows, cols) == tile and (kp > 1) == split
+    print(f"case: {M} x {K} x {Ns} gs {gs} {bits}-bit {dtype}", flush=True)
+    dt = torch.bfloat16 if dtype == "bf16" else torch.float16
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(M + K + gs + bits)
+    x = torch.randn((M, K), generator=gen, device=dev).to(dt)
+    mats = [_random_weights(dev, gen, N, K, gs, bits, dt) for N in Ns]
+    if len(Ns) > 1:
+        ys = vq.quantized_matmul_multi(x, mats, group_size=gs, bits=bits)
+    else:
+        ys = [vq.quantized_matmul(x, *mats[0], group_size=gs, bits=bits)]
+    for y, mat in zip(ys, mats):
+        _within(y, x, mat, gs, bits)
 
 
 def test_tables_and_workspaces(dev):
