@@ -32,9 +32,13 @@
 // and 64 x 256 with three stages and one workgroup per CU 300 us (the
 // general kernel of 32-row blocks, which this one replaces: 1.6 ms).
 //
+// Two workgroups share a CU's LDS (three of the 32 x 128 tile); with 8-bit
+// weights the stages of the larger tiles take it for one.
+//
 // The loop is software-pipelined by hand (unit()): left to itself the
 // compiler hoists reads and products until it spills, and a spill's reload
-// waits for the DMA in flight.
+// waits for the DMA in flight.  What still spills (bytes per lane): the 96 x
+// 128 tile 12..28, at group size 32 it and the 64 x 256 one 108..224.
 #pragma once
 
 #include "dfmi_device.h"

@@ -6,9 +6,11 @@
 
 namespace dfmi {
 
-// The tiles, and what the plan chooses by: the time of one 128-k step of a
-// workgroup alone on its CU (us), its share per workgroup of the CU's time
-// with `slots` of them on every CU.
+// The tiles, and what the plan chooses by, in us per 128-k step: `full`, a
+// workgroup's share of a CU's time while whole rounds of 256 * slots of them
+// follow each other (the next workgroups already run on the CU), and `alone`,
+// the step of the last, partly filled round.  slots says how many workgroups
+// a round puts on a CU, not how many the CU holds.
 struct GemmCfg {
   int bm, bn, slots;
   double alone, full;
@@ -34,6 +36,9 @@ struct GemmPlan {
 // eight K x N from 1024 x 512 to 17408 x 5120, MI355X, gs 64, 4-bit, bf16):
 // what the rule picks is 1.2 % slower in the mean than the best of them all,
 // 14 % at worst; 64 x 128, 32 x 256 and 128 x 256 tiles would add 0.9 %.
+// Known limits: a single whole round is priced at `full` although its
+// workgroups have no successors, so 256 of them are estimated below 255; and
+// 8-bit weights, groups of 32 (which spill) and f16 take the same figures.
 static GemmPlan gemm_plan(int64_t M, int64_t K, const int64_t* Ns, int nseg,
                           size_t max_partials) {
   const int steps = (int)((K + kGemmK - 1) / kGemmK);

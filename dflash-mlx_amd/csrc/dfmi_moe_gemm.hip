@@ -184,7 +184,8 @@ int moe_segments_launch(const int32_t* rhs, int P, int32_t* segs, hipStream_t st
 // Units of (segment, 128 table columns): 128 weight rows of the expert, or
 // for the SwiGLU 64 output columns, whose gate and up rows alternate 32 at a
 // time, as the interleaved table does: wavefront w takes gate (even w) or up
-// rows.  Three workgroups per CU (45 KB of LDS, at most 168 VGPRs) take
+// rows.  Three workgroups per CU (45 KB of LDS, 168 VGPRs and 24 bytes of
+// spills per lane) take
 // consecutive units, those of an XCD a contiguous eighth, so a segment's units
 // share its activations, and an expert's segments its weights, in one L2.
 //

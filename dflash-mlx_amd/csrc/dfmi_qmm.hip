@@ -499,8 +499,9 @@ static int plan_stream(int64_t M, int64_t K, int64_t N, int gs, int bits,
     // ranges -- 5120 x 34816 24.5 vs 26.7 us, 17408 x 5120 15.6 vs 17.2 us,
     // 5120 x 151936 95.5 vs 102.7 us -- and loses on short ones: 5120 x
     // 5120 9.6 vs 9.0 us, 4096 x 4096 8.7 vs 7.9 us)
-    // (two activation blocks: 64-row blocks only, two stages of 25 KB, three
-    // workgroups per CU)
+    // (two activation blocks: 64-row blocks only, of 25 KB stages: three of
+    // them and two workgroups per CU on grids of at most 512, else two and
+    // three)
     int rw = rows == 128 ? 2 : 1;
     if (rows == 0 && geo.nb128 && kAutoRows128 && mt == 1) {
       StreamPlan q;

@@ -151,7 +151,7 @@ def test_gather_pairs_invalid_ids_give_nan_rows(dev, glu):
 @pytest.mark.parametrize("P", [1, 256, 257])
 def test_gather_pairs_pair_counts(dev, P):
     """One pair (one unit per column block, two workgroups), the 256-pair
-    limit of the kernel's LDS tables, and 257 pairs (the plain main loops)."""
+    limit of the kernel's LDS tables, and 257 pairs (32-row matrix-core tiles)."""
     E, N, K, R = 64, 128, 512, 32
     gate = _experts(E, N, K, 64, "bf16", seed=P)
     up = _experts(E, N, K, 64, "bf16", seed=P + 1)

@@ -72,7 +72,7 @@ def _multi(dev, x, mats, gs, dtype="bf16", bits=4):
     (4, 2048, (100, 3000, 64, 7), "qmm_stream_multi_kernel"),    # ragged, four matrices
     (32, 2048, (300, 0, 700), "qmm_stream_multi_kernel"),        # two activation blocks; empty matrix
     (16, 1024, (65,), "qmm_stream_kernel"),
-    (40, 2048, (512, 256), None),                                # M > 32: one call per matrix
+    (40, 2048, (512, 256), None),                                # M > 32: one matrix-core launch
     (16, 1088, (640, 256), None)])                               # K % 256 != 0: one call per matrix
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
 def test_multi_matches_oracle_and_separate_calls(dev, M, K, Ns, kernel, dtype):
