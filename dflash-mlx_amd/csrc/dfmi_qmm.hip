@@ -980,8 +980,9 @@ static int launch_streaming(const void* x, int x_dtype, const StreamSegs& segs, 
 
 // One matrix-core launch of two or three matrices: each takes that kernel and
 // starts on a 16-byte boundary of a table of them all.  (A layer's q/k/v, o,
-// gate/up and down over 77 rows of 5120, 17408 wide: 144 us, with a launch for
-// each matrix 163: fewer nearly empty last waves and split sums.)
+// gate/up and down over 77 rows of 5120, 17408 wide, with tables at hand: 144
+// us, with a launch for each matrix 163: fewer nearly empty last waves and
+// split sums.)
 static bool use_gemm_multi(int64_t M, int64_t K, const int64_t* Ns, int nseg, int gs) {
   if (nseg < 2 || nseg > 3) return false;
   int64_t sum = 0;

@@ -8,7 +8,8 @@
  * memory and none keeps a pointer past its return (dfmi_qmm_prepare writes
  * the pointers it is given into the caller's record buffer, which
  * dfmi_qmm_run then reads).  Functions are reentrant;
- * the process state is the thread-local error string and, for
+ * the process state is the thread-local error string, a lock held while a
+ * call with a workspace enqueues its kernels and, for
  * dfmi_qmm_affine_noalloc only, its static device scratch array and the
  * per-device address of it (set once, under a lock).
  *

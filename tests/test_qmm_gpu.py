@@ -232,7 +232,7 @@ def test_unsupported_raises(dev):
     (16, 512, 16448, 64),   # streaming, 4 wavefronts (257 blocks), unsplit
     (16, 4096, 12288, 64),  # streaming, 4 wavefronts in two stages, K split 2 ways (the 9B gate/up plan)
     (16, 2048, 12288, 64),  # the same plan at 4 steps per split
-    (33, 256, 40, 64),      # register-load kernel (M > 32)
+    (33, 256, 40, 64),      # matrix-core kernel (M > 32)
     (1, 96, 16, 32)])       # register-load kernel (K not whole 256-k steps)
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
 def test_8bit_matches_oracle(dev, M, K, N, gs, dtype):
