@@ -871,7 +871,7 @@ using namespace dfmi;
 // Automatic choice (measured on MI355X): the streaming kernel is faster on
 // every shape it takes; beyond 32 rows qmm_gemm_kernel (use_gemm), and the
 // general kernel covers the rest (K not a multiple of 256 or of 8 groups,
-// weights over 2 GiB).
+// weights over 2 GiB, small products beyond 32 rows).
 static bool use_stream(int64_t M, int64_t K, int64_t N, int gs, int bits,
                        const dfmi_qmm_tuning* tune) {
   const int path = tune ? tune->path : 0;
@@ -1009,10 +1009,23 @@ static int64_t multi_stream_cols(int64_t M, int64_t K, const int64_t* Ns, int ns
 }
 
 // The matrix-core kernel for many rows is the automatic choice above the
-// streaming kernels' 32 rows (a forced general plan keeps the general kernel).
-static bool use_gemm(int64_t M, int64_t K, int64_t N, int gs, const dfmi_qmm_tuning* tune) {
-  return gemm_shape(M, K, N, gs) &&
-         (!tune || (tune->path == 0 && !tune->tiles_per_wave && !tune->waves_per_block));
+// streaming kernels' 32 rows (a forced general plan keeps the general kernel),
+// but for small products: there the general kernels, one launch with no table
+// to build and no scratch, take no longer.  Their time is a row block's chain
+// along K (4096: 12.6 us, 8192: 22) or, past a chip full of them, the product's
+// size.  Measured over M 33..333, 29 K x N, both sides with what they launch,
+// us on the GPU / per call of a Python loop: 33 x 512 x 256 4.1 / 12 against
+// 7.8 / 17; 128 x 4096 x 1024 12.9 / 13 against 13.3 / 17; beyond the line 200 x
+// 2048 x 2048 20 / 20 against 15 / 17, 8-bit 96 x 2048 x 2048 20 / 21 against 13
+// / 17, and 33 x 8192 x 1024 22 / 23 against 14 / 17.
+static bool use_gemm(int64_t M, int64_t K, int64_t N, int gs, int bits,
+                     const dfmi_qmm_tuning* tune) {
+  if (!gemm_shape(M, K, N, gs) ||
+      (tune && (tune->path != 0 || tune->tiles_per_wave || tune->waves_per_block)))
+    return false;
+  const int64_t block = bits == 4 ? 32 : 16;  // the general kernels' row blocks
+  const int64_t size = (M + block - 1) / block * block * N * K;
+  return K > 4096 || size > (bits == 4 ? 1ll << 29 : 1ll << 28);
 }
 
 extern "C" size_t dfmi_qmm_workspace_bytes_ex(int64_t M, int64_t K, int64_t N, int group_size,
@@ -1020,7 +1033,7 @@ extern "C" size_t dfmi_qmm_workspace_bytes_ex(int64_t M, int64_t K, int64_t N, i
   if (validate_qmm(DFMI_BF16, M, K, N, group_size, bits) != DFMI_OK || M == 0 || N == 0 ||
       !valid_path(tuning))
     return 0;
-  if (use_gemm(M, K, N, group_size, tuning)) return gemm_workspace_bytes(M, K, N, group_size);
+  if (use_gemm(M, K, N, group_size, bits, tuning)) return gemm_workspace_bytes(M, K, N, group_size);
   if (!use_stream(M, K, N, group_size, bits, tuning)) return 0;
   StreamPlan p;
   if (plan_stream(M, K, N, group_size, bits, tuning, p) != DFMI_OK) return 0;
@@ -1074,7 +1087,7 @@ extern "C" int dfmi_qmm_gemm_plan(int64_t M, int64_t K, const int64_t* Ns, int n
     if (rc != DFMI_OK) return rc;
   }
   *tile_rows = *tile_cols = *k_splits = 0;
-  if (nseg == 1 ? Ns[0] > 0 && use_gemm(M, K, Ns[0], group_size, nullptr)
+  if (nseg == 1 ? Ns[0] > 0 && use_gemm(M, K, Ns[0], group_size, bits, nullptr)
                 : use_gemm_multi(M, K, Ns, nseg, group_size))
     gemm_plan_query(M, K, Ns, nseg, tile_rows, tile_cols, k_splits);
   return DFMI_OK;
@@ -1084,7 +1097,7 @@ extern "C" const char* dfmi_qmm_kernel_name(int64_t M, int64_t K, int64_t N, int
                                              int bits, const dfmi_qmm_tuning* tuning) {
   if (validate_qmm(DFMI_BF16, M, K, N, group_size, bits) != DFMI_OK || !valid_path(tuning))
     return nullptr;
-  if (use_gemm(M, K, N, group_size, tuning)) return "qmm_gemm_kernel";
+  if (use_gemm(M, K, N, group_size, bits, tuning)) return "qmm_gemm_kernel";
   if (bits == 8) return use_stream(M, K, N, group_size, bits, tuning) ? "qmm8_stream_kernel"
                                                                       : "qmm8_kernel";
   return use_stream(M, K, N, group_size, bits, tuning) ? "qmm_stream_kernel" : "qmm_dense_kernel";
@@ -1125,7 +1138,7 @@ static int qmm_affine(const void* x, int x_dtype, const uint32_t* w_q, const voi
     return DFMI_EINVAL;
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (use_gemm(M, K, N, group_size, tuning)) {
+  if (use_gemm(M, K, N, group_size, bits, tuning)) {
     const dfmi_qmm_segment seg{w_q, scales, biases, y, N, sb_pairs};
     rc = gemm_launch(x, x_dtype, &seg, 1, nullptr, sb_stride, M, K, group_size, bits, workspace,
                      workspace_bytes, st);
@@ -1282,7 +1295,7 @@ extern "C" int dfmi_qmm_affine_noalloc(const void* x, int x_dtype, const uint32_
   if (M == 0 || N == 0) return DFMI_OK;
   // more rows than the streaming kernels take: the general kernel, which
   // needs no scratch (so such calls may overlap)
-  if (use_gemm(M, K, N, group_size, nullptr))
+  if (use_gemm(M, K, N, group_size, bits, nullptr))
     return dfmi_qmm_affine_ex(x, x_dtype, w_q, scales, biases, y, M, K, N, group_size, bits,
                               nullptr, 0, nullptr, stream);
   const size_t need = dfmi_qmm_workspace_bytes_ex(M, K, N, group_size, bits, nullptr);

@@ -20,7 +20,8 @@ pass over both weight sets), and the weighted sum is ``dfmi_moe_combine``.
 Where the expert shapes allow (4-bit, gs 64 / 128, K a multiple of 256,
 N a multiple of 128, or 64 for the SwiGLU pair) the
 gathers take the experts' (scale, bias) pair table (``dfmi_moe_pairs``,
-built once per weight set and cached, or beyond 256 pairs in each call) and the stream's gather workspace, and
+built once per weight set and cached, or beyond 256 pairs in each call that it
+pays for) and the stream's gather workspace, and
 run the pair-streaming main loop (``dfmi_gather_qmm_*_pairs``); otherwise,
 and during graph capture before a table exists, the plain entry points.
 """
@@ -58,13 +59,13 @@ def _expert_weights(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
 
 def _pairs_table(pairs: Optional[torch.Tensor], scales: torch.Tensor, biases: torch.Tensor,
                  up: Optional[Tuple[torch.Tensor, torch.Tensor]], K: int, N: int,
-                 group_size: int, bits: int, use_pairs: bool, few: bool):
+                 group_size: int, bits: int, use_pairs: bool, P: int, few: bool):
     """The experts' pair table (``dfmi_moe_pairs`` layout), or None.
 
     An explicit table is checked for shape and device; otherwise, where the
     shape takes one, it is the cached table of these scales / biases (few
-    pairs: built on first use, never during graph capture) or one built for
-    the call from the scales as they are (many pairs)."""
+    pairs: built on first use, never during graph capture) or, for many pairs,
+    one built for the call from the scales as they are, where that pays."""
     E, _, G = (int(d) for d in scales.shape)
     cols = 2 * N if up is not None else N
     if pairs is not None:
@@ -77,6 +78,8 @@ def _pairs_table(pairs: Optional[torch.Tensor], scales: torch.Tensor, biases: to
         return None
     if few:
         return _runtime.PAIRS.get(scales, biases, up, experts=True)
+    if not _table_pays(P, K, N, E, group_size, up is not None):
+        return None
     return _runtime.build_moe_pairs(scales, biases, *(up if up is not None else ()))
 
 
@@ -90,6 +93,22 @@ def _stream_table(x_rows: int, P: int, K: int, N: int, E: int) -> bool:
     ``moe_gemm_kernel``."""
     return (P <= 256 and x_rows <= 32767 and E < 65535 and x_rows * K < 1 << 30
             and N * K < 1 << 32 and P * N < 1 << 30)
+
+
+def _table_pays(P: int, K: int, N: int, E: int, group_size: int, swiglu: bool) -> bool:
+    """Many pairs: whether 32-row tiles reading a table built for the call beat
+    the gathers that read the scales in place, one launch.  Measured over 8 .. 256
+    experts, 257 .. 4096 sorted pairs, us on the GPU: SwiGLU of 512 x 2048 (the
+    persistent gather) 1000 pairs of 256 experts 85 against 92, 1536 148 against
+    95; 768 x 2048, 64 experts, 512 pairs 36 against 36, 1024 51 against 37; down
+    2048 x 512 of 256 experts (a workgroup per run) 257 pairs 35 against 39, 512 48
+    against 47, 4096 106 against 59; 1024 x 512 of 8 experts 257 pairs 13.5 against
+    13.2, 1024 42 against 17.  (Per call of a Python loop the table adds 10 us
+    where the GPU is not the limit, so a tie goes to the gathers.)"""
+    size = P * N * K * (2 if swiglu else 1)
+    if P <= 1024 and K >= 1024 and K % 512 == 0 and K // group_size <= 32:
+        return P * N * K > 1 << 30
+    return size >= 1 << 29 or (P >= 64 * E and size >= 1 << 27)
 
 
 def _space(lib, device: torch.device, table, few: bool):
@@ -135,7 +154,7 @@ def gather_qmm(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: t
         raise ValueError("lhs_indices and rhs_indices must have the same length")
     y = torch.empty((P, N), dtype=x.dtype, device=x.device)
     few = _stream_table(int(x2.shape[0]), P, K, N, E)
-    table = _pairs_table(pairs, scales, biases, None, K, N, group_size, bits, use_pairs, few)
+    table = _pairs_table(pairs, scales, biases, None, K, N, group_size, bits, use_pairs, P, few)
     lib = _lib.load()
     ws, ws_bytes, _scratch = _space(lib, x.device, table, few)
     _lib.check(lib.dfmi_gather_qmm_affine_pairs(
@@ -167,7 +186,7 @@ def gather_swiglu(x: torch.Tensor, gate: Triple, up: Triple, rhs_indices: torch.
     P = int(rhs.shape[0])
     h = torch.empty((P, N), dtype=x.dtype, device=x.device)
     few = _stream_table(int(x2.shape[0]), P, K, N, Eg)
-    table = _pairs_table(pairs, sg, bg, (su, bu), K, N, group_size, bits, use_pairs, few)
+    table = _pairs_table(pairs, sg, bg, (su, bu), K, N, group_size, bits, use_pairs, P, few)
     lib = _lib.load()
     ws, ws_bytes, _scratch = _space(lib, x.device, table, few)
     _lib.check(lib.dfmi_gather_qmm_swiglu_pairs(
@@ -218,8 +237,9 @@ def _switch_glu(x, inds, gate: Triple, up: Triple, down: Triple, group_size: int
     The pair order lies in scratch of the call's own."""
     _runtime.require_device(x, "x")
     dev = x.device
+    index = x.get_device()
     for t in (inds, *gate, *up, *down):
-        if t.device != dev:
+        if t.get_device() != index:
             raise ValueError(f"x is on {dev}, expert ids or weights on {t.device}")
     T, k = int(inds.shape[0]), int(inds.shape[1])
     D = int(x.shape[-1])
@@ -238,8 +258,8 @@ def _switch_glu(x, inds, gate: Triple, up: Triple, down: Triple, group_size: int
     h = torch.empty((P, I), dtype=x.dtype, device=dev)
     y = torch.empty((P, D), dtype=x.dtype, device=dev)
     few = _stream_table(T, P, D, I, E) and _stream_table(P, P, I, D, E)
-    glu = _pairs_table(None, sg, bg, (su, bu), D, I, group_size, bits, True, few)
-    dn = _pairs_table(None, sd, bd, None, I, D, group_size, bits, True, few)
+    glu = _pairs_table(None, sg, bg, (su, bu), D, I, group_size, bits, True, P, few)
+    dn = _pairs_table(None, sd, bd, None, I, D, group_size, bits, True, P, few)
     gws, gws_bytes, _gather = _space(lib, dev, (glu if glu is not None else dn) if few else None,
                                      few)
     _lib.check(lib.dfmi_switch_glu(

@@ -99,7 +99,9 @@ typedef struct dfmi_qmm_tuning {
  * on scheduling: every K split is summed in a fixed order.  Shapes that split
  * K across workgroups need the workspace dfmi_qmm_workspace_bytes reports
  * (0 bytes -> workspace may be NULL); it must be zero-filled when created.
- * With more than 32 rows the workspace is optional: the matrix-core kernel
+ * With more than 32 rows small products (up to about 2^29 multiply-adds, 2^28
+ * at 8 bits, K up to 4096) run on the general kernels, without a workspace.
+ * For the others the workspace is optional: the matrix-core kernel
  * keeps the partial tiles of a K split in it, and the pair table where the
  * call brings none; with less of it the call runs unsplit, or on the general
  * kernel (the sums of another split are in another fp32 order).

@@ -53,6 +53,7 @@ def library(monkeypatch):
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
     monkeypatch.setattr(_runtime.PAIRS, "get", lambda *a, **k: torch.zeros(1))
     monkeypatch.setattr(_runtime, "WORKSPACES", _runtime._WorkspaceCache())
+    monkeypatch.setattr(moe, "_table_pays", lambda *a: True)
     return use
 
 
@@ -132,6 +133,17 @@ def _from_two_threads(calls, check):
     assert not errors, errors[0]
 
 
+def test_where_a_table_for_many_pairs_pays():
+    """The rule's lines: the persistent gather's shapes, the others by size, and
+    long runs of few experts."""
+    pays = moe._table_pays
+    assert not pays(1024, 2048, 512, 256, 64, True) and pays(1025, 2048, 512, 256, 64, True)
+    assert not pays(512, 2048, 768, 64, 64, True) and pays(1024, 2048, 768, 64, 64, True)
+    assert not pays(511, 512, 2048, 256, 64, False) and pays(512, 512, 2048, 256, 64, False)
+    assert pays(512, 512, 1024, 8, 64, False) and not pays(512, 512, 1024, 64, 64, False)
+    assert not pays(257, 256, 128, 1, 64, False)
+
+
 def test_tables_are_waited_for_once_per_stream(monkeypatch):
     """A table is waited for on the device by the first call on each stream but
     the one that built it, never while capturing, and its event not queried."""
@@ -165,13 +177,18 @@ def test_tables_are_waited_for_once_per_stream(monkeypatch):
 def test_expert_tensors_on_another_device(library):
     """switch_glu refuses expert ids or weights that are not where x is, before
     anything reaches the library."""
+    class Elsewhere(torch.Tensor):
+        def get_device(self):
+            return 1
+
     gate, down = _weights(128, 256, lead=(4,)), _weights(256, 128, lead=(4,))
     x, ids = torch.zeros((16, 256), dtype=torch.bfloat16), torch.zeros((16, 8), dtype=torch.int32)
     for at in range(10):
         lib = library("dfmi_switch_glu", ())
         lib.second.set()
-        ts = [t.to("meta") if i == at else t for i, t in enumerate((ids, *gate, *gate, *down))]
-        with pytest.raises(ValueError, match="on meta"):
+        ts = [t.as_subclass(Elsewhere) if i == at else t
+              for i, t in enumerate((ids, *gate, *gate, *down))]
+        with pytest.raises(ValueError, match="expert ids or weights on"):
             moe._switch_glu(x, ts[0], ts[1:4], ts[4:7], ts[7:10], 64, 4)
         assert not lib.seen
 
@@ -227,7 +244,7 @@ def test_threads_on_one_stream(dev, shared):
     """K splits (product, then sum) from two threads on one stream, through
     the operator and through the C ABI with one workspace for both: each call
     has its own result."""
-    M, K, Ns, gs = 40, 4096, (256, 512), 64
+    M, K, Ns, gs = 40, 8192, (256, 512), 64
     gen = torch.Generator(device=dev)
     gen.manual_seed(2)
 

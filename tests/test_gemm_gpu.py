@@ -1,5 +1,6 @@
-"""GPU parity of ``qmm_gemm_kernel`` (more than 32 activation rows).  The small
-shapes, against the CPU oracle, are planned on its 32 x 128 tile;
+"""GPU parity of ``qmm_gemm_kernel`` (more than 32 activation rows; small
+products with K up to 4096 stay on the general kernels).  The shapes of few
+rows and columns, against the CPU oracle, are planned on its 32 x 128 tile;
 ``test_every_tile`` takes each of the three tiles (32 x 128, 96 x 128, 64 x
 256), with one and several K splits, ragged rows, columns and K, against
 float64 sums, and checks which tile the plan took.
@@ -43,9 +44,9 @@ def _check(got, case, gs, bits, dtype):
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("M,K,N,gs", [
-    (33, 32, 1, 32), (33, 64, 4, 64), (64, 128, 127, 128), (65, 160, 128, 32),
-    (77, 192, 129, 64), (96, 1088, 260, 64), (97, 1152, 1000, 128), (129, 320, 256, 32),
-    (200, 576, 2501, 64), (65, 4096, 300, 64),
+    (33, 4128, 1, 32), (33, 4160, 4, 64), (64, 4224, 127, 128), (65, 4256, 128, 32),
+    (77, 4288, 129, 64), (96, 5184, 260, 64), (97, 5248, 1000, 128), (129, 4416, 256, 32),
+    (200, 4672, 2501, 64), (65, 8192, 300, 64),
 ])
 def test_tile_edges(dev, M, K, N, gs, bits, dtype):
     from dflash_mlx_amd import _lib, verify_qmm as vq
@@ -56,6 +57,32 @@ def test_tile_edges(dev, M, K, N, gs, bits, dtype):
     _check(from_dev(y, dtype), case, gs, bits, dtype)
     again = vq.quantized_matmul(x, w, s, b, group_size=gs, bits=bits)
     assert np.array_equal(from_dev(y, dtype), from_dev(again, dtype))
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("M,K,N,gs", [
+    (33, 32, 1, 32), (33, 64, 4, 64), (64, 128, 127, 128), (77, 192, 129, 64), (97, 1152, 1000, 128),
+    (333, 4096, 40, 64), (64, 4096, 1024, 64), (64, 4096, 1028, 64), (256, 512, 2048, 32),
+])
+def test_small_products_on_the_general_kernels(dev, M, K, N, gs, bits, dtype):
+    """Up to the line of the dispatch, and past it at 8 bits: one launch without
+    a workspace, the bits of the forced general plan."""
+    import torch
+
+    from dflash_mlx_amd import _lib, verify_qmm as vq
+
+    lib, rows = _lib.load(), -(-M // 16) * 16 if bits == 8 else -(-M // 32) * 32
+    small = rows * K * N <= (1 << 28 if bits == 8 else 1 << 29)
+    name = lib.dfmi_qmm_kernel_name(M, K, N, gs, bits, None)
+    assert (name != b"qmm_gemm_kernel") == small
+    assert (lib.dfmi_qmm_workspace_bytes(M, K, N, gs, bits) == 0) == small
+    case, (x, w, s, b) = _case(dev, M, K, N, gs, bits, dtype, seed=M + K + N + bits)
+    y = vq.quantized_matmul(x, w, s, b, group_size=gs, bits=bits)
+    _check(from_dev(y, dtype), case, gs, bits, dtype)
+    if small:
+        assert torch.equal(y, vq.quantized_matmul(x, w, s, b, group_size=gs, bits=bits,
+                                                  tuning=_lib.QmmTuning(1, 0, 0, 0)))
 
 
 def _plan(M, K, Ns, gs, bits):
@@ -99,12 +126,12 @@ def _within(y, x, mat, gs, bits):
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("gs", [32, 64, 128])
 @pytest.mark.parametrize("tile,split,M,K,Ns", [
-    ((32, 128), False, 65, 192, (129,)), ((32, 128), True, 65, 1088, (136,)),
-    ((32, 128), True, 500, 4160, (644, 4, 640)),
-    ((64, 256), False, 103, 64, (16388,)), ((64, 256), False, 1000, 192, (2504,)),
-    ((64, 256), False, 1000, 64, (2501,)), ((64, 256), True, 97, 2112, (8200,)),
+    ((32, 128), False, 1000, 576, (1000,)), ((32, 128), False, 97, 1088, (4100,)),
+    ((32, 128), True, 65, 4288, (136,)), ((32, 128), True, 500, 4160, (644, 4, 640)),
+    ((64, 256), False, 103, 320, (16388,)), ((64, 256), False, 1000, 320, (2504,)),
+    ((64, 256), False, 1000, 576, (2501,)), ((64, 256), True, 97, 2112, (8200,)),
     ((64, 256), True, 500, 4160, (1284,)), ((64, 256), False, 1000, 192, (1028, 4, 1480)),
-    ((96, 128), False, 229, 64, (16388,)), ((96, 128), False, 500, 192, (8200,)),
+    ((96, 128), False, 229, 192, (16388,)), ((96, 128), False, 500, 192, (8200,)),
     ((96, 128), True, 77, 4160, (12296,)), ((96, 128), True, 65, 4160, (6148, 4, 6148)),
 ])
 def test_every_tile(dev, tile, split, M, K, Ns, gs, bits, dtype):
@@ -140,7 +167,7 @@ def test_tables_and_workspaces(dev):
     from dflash_mlx_amd import _lib, _runtime
 
     lib = _lib.load()
-    M, K, N, gs = 77, 2048, 520, 64
+    M, K, N, gs = 77, 6144, 520, 64
     case, (x, w, s, b) = _case(dev, M, K, N, gs, 4, "bf16", seed=5)
     need = int(lib.dfmi_qmm_workspace_bytes(M, K, N, gs, 4))
     ws = torch.zeros(need + 256, dtype=torch.uint8, device=dev)
@@ -182,10 +209,10 @@ def test_rows_with_infinities_stay_apart(dev):
 
     from dflash_mlx_amd import verify_qmm as vq
 
-    M, K, N, gs = 70, 448, 256, 64
+    M, K, N, gs = 70, 4544, 256, 64
     _, (x, w, s, b) = _case(dev, M, K, N, gs, 4, "bf16", seed=9)
     ref = vq.quantized_matmul(x, w, s, b, group_size=gs, bits=4)
-    x[11, 5], x[40, 447], x[69, 0] = float("inf"), float("nan"), -float("inf")
+    x[11, 5], x[40, 4543], x[69, 0] = float("inf"), float("nan"), -float("inf")
     got = vq.quantized_matmul(x, w, s, b, group_size=gs, bits=4)
     rows = [r for r in range(M) if r not in (11, 40, 69)]
     assert torch.equal(got[rows], ref[rows])
@@ -343,7 +370,7 @@ def test_scales_are_read_at_each_call(dev, route):
 
     from dflash_mlx_amd import verify_linear as vl, verify_qmm as vq
 
-    M, K, Ns, gs = 45, 2048, (384, 256), 64
+    M, K, Ns, gs = 45, 6144, (384, 256), 64
     mats, x = [], None
     for i, N in enumerate(Ns):
         _, (xi, w, s, b) = _case(dev, M, K, N, gs, 4, "bf16", seed=70 + i)

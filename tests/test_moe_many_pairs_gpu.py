@@ -1,5 +1,5 @@
-"""GPU parity of the routed experts beyond 256 pairs (``moe_gemm_kernel``) and
-of the device sort of ``switch_glu``, against a float64 torch restatement that
+"""GPU parity of the routed experts beyond 256 pairs (``moe_gemm_kernel``, and the
+gathers that take the smaller of them) and of the device sort of ``switch_glu``, against a float64 torch restatement that
 rounds where mlx-lm's operators do.  Tolerance: the reference's own metric,
 max|d| / (max|ref| + 1e-3) <= 1e-2 (tests/test_verify_qmm_parity.py:69-70)."""
 
@@ -63,13 +63,23 @@ SHAPES = [
 ]
 
 
+@pytest.fixture
+def pays(monkeypatch):
+    """Decide for the rule whether many pairs get a table."""
+    from dflash_mlx_amd import moe
+
+    return lambda answer: monkeypatch.setattr(moe, "_table_pays", lambda *a: answer)
+
+
+@pytest.mark.parametrize("table", [True, False])
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
 @pytest.mark.parametrize("T,k,E,D,I,gs", SHAPES)
-def test_switch_glu(dev, T, k, E, D, I, gs, dtype):
+def test_switch_glu(dev, pays, T, k, E, D, I, gs, dtype, table):
     import torch
 
     from dflash_mlx_amd import moe
 
+    pays(table)
     dt = torch.bfloat16 if dtype == "bf16" else torch.float16
     gen = torch.Generator(device=dev)
     gen.manual_seed(T + E + D)
@@ -90,14 +100,16 @@ def test_switch_glu(dev, T, k, E, D, I, gs, dtype):
     assert torch.equal(y.view(torch.int16), y2.view(torch.int16))
 
 
+@pytest.mark.parametrize("table", [True, False])
 @pytest.mark.parametrize("ordered", [False, True])
-def test_gathers_many_pairs(dev, ordered):
+def test_gathers_many_pairs(dev, pays, ordered, table):
     """gather_swiglu / gather_qmm on 1100 pairs, sorted and not, with row ids
     out of range: each pair's row as the reference has it."""
     import torch
 
     from dflash_mlx_amd import moe
 
+    pays(table)
     gen = torch.Generator(device=dev)
     gen.manual_seed(3)
     E, D, I, P, R, gs = 20, 512, 256, 1100, 90, 64
@@ -120,13 +132,14 @@ def test_gathers_many_pairs(dev, ordered):
     _close(torch, y[ok], yr[ok])
 
 
-def test_switch_glu_captured(dev):
+def test_switch_glu_captured(dev, pays):
     """Captured before and after the stream has its tables and workspaces,
     replayed with new routing: the eager results."""
     import torch
 
     from dflash_mlx_amd import moe
 
+    pays(True)
     gen = torch.Generator(device=dev)
     gen.manual_seed(8)
     E, D, I, gs = 16, 256, 128, 64
@@ -153,13 +166,15 @@ def test_switch_glu_captured(dev):
             _close(torch, y, yr)
 
 
-def test_scales_are_read_at_each_call(dev):
+@pytest.mark.parametrize("table", [True, False])
+def test_scales_are_read_at_each_call(dev, pays, table):
     """Beyond 256 pairs the results are of the scales as they are: after an
     update that counts no version, and in a graph replayed after one."""
     import torch
 
     from dflash_mlx_amd import moe
 
+    pays(table)
     gen = torch.Generator(device=dev)
     gen.manual_seed(12)
     E, D, I, gs = 16, 256, 128, 64

@@ -143,7 +143,8 @@ def test_siblings_over_eager_calls_and_two_captures(dev, M):
         g = gate(x)
     for _ in range(3):
         x.copy_(torch.randn((M, K), generator=gen, device=dev).to(torch.bfloat16))
-        want_g, want_u = gate(x.clone()), up(x.clone())
+        same = x.clone()  # one shared launch for both
+        want_g, want_u = gate(same), up(same)
         for graph, y, want in ((graphs[1], g, want_g), (graphs[0], u, want_u)):
             y.fill_(float("nan"))
             graph.replay()
