@@ -978,19 +978,38 @@ static int launch_streaming(const void* x, int x_dtype, const StreamSegs& segs, 
   return run_streaming(L, x, st);
 }
 
+// Beyond 32 rows (a gemm_shape), products that the general kernels, one launch
+// with no table to build and no scratch, take no longer over than the
+// matrix-core kernel.  Their time is a row block's chain along K (4096: 12.6 us,
+// 8192: 22) or, past a chip full of them, the product's size.  Measured over M
+// 33..333, 29 K x N, both sides with what they launch, us on the GPU / per call
+// of a Python loop: 33 x 512 x 256 4.1 / 12 against 7.8 / 17; 128 x 4096 x 1024
+// 12.9 / 13 against 13.3 / 17; beyond the line 200 x 2048 x 2048 20 / 20 against
+// 15 / 17, 8-bit 96 x 2048 x 2048 20 / 21 against 13 / 17, and 33 x 8192 x 1024 22 /
+// 23 against 14 / 17.
+static bool small_product(int64_t M, int64_t K, int64_t N, int bits) {
+  const int64_t block = bits == 4 ? 32 : 16;  // the general kernels' row blocks
+  return K <= 4096 && (M + block - 1) / block * block * N * K <=
+                          (bits == 4 ? 1ll << 29 : 1ll << 28);
+}
+
 // One matrix-core launch of two or three matrices: each takes that kernel and
 // starts on a 16-byte boundary of a table of them all.  (A layer's q/k/v, o,
 // gate/up and down over 77 rows of 5120, 17408 wide, with tables at hand: 144
 // us, with a launch for each matrix 163: fewer nearly empty last waves and
-// split sums.)
-static bool use_gemm_multi(int64_t M, int64_t K, const int64_t* Ns, int nseg, int gs) {
+// split sums.)  Two small products of short K are two launches: 33 x 512 x (256,
+// 256) 8-bit 7.7 us against 9.3, 33 x 768 x (1000, 1000) 9.8 against 10.8; K =
+// 1024 and three matrices are not (33 x 512 x (512, 128, 128) 12 against 9.5).
+static bool use_gemm_multi(int64_t M, int64_t K, const int64_t* Ns, int nseg, int gs, int bits) {
   if (nseg < 2 || nseg > 3) return false;
   int64_t sum = 0;
   for (int i = 0; i < nseg; ++i) {
     if (Ns[i] < 1 || Ns[i] % 4) return false;
     sum += Ns[i];
   }
-  return gemm_shape(M, K, sum, gs);
+  return gemm_shape(M, K, sum, gs) &&
+         !(nseg == 2 && K <= 768 && small_product(M, K, Ns[0], bits) &&
+           small_product(M, K, Ns[1], bits));
 }
 
 // Shared-activation launches take the streaming kernel when every matrix
@@ -1010,22 +1029,12 @@ static int64_t multi_stream_cols(int64_t M, int64_t K, const int64_t* Ns, int ns
 
 // The matrix-core kernel for many rows is the automatic choice above the
 // streaming kernels' 32 rows (a forced general plan keeps the general kernel),
-// but for small products: there the general kernels, one launch with no table
-// to build and no scratch, take no longer.  Their time is a row block's chain
-// along K (4096: 12.6 us, 8192: 22) or, past a chip full of them, the product's
-// size.  Measured over M 33..333, 29 K x N, both sides with what they launch,
-// us on the GPU / per call of a Python loop: 33 x 512 x 256 4.1 / 12 against
-// 7.8 / 17; 128 x 4096 x 1024 12.9 / 13 against 13.3 / 17; beyond the line 200 x
-// 2048 x 2048 20 / 20 against 15 / 17, 8-bit 96 x 2048 x 2048 20 / 21 against 13
-// / 17, and 33 x 8192 x 1024 22 / 23 against 14 / 17.
+// but for small products.
 static bool use_gemm(int64_t M, int64_t K, int64_t N, int gs, int bits,
                      const dfmi_qmm_tuning* tune) {
-  if (!gemm_shape(M, K, N, gs) ||
-      (tune && (tune->path != 0 || tune->tiles_per_wave || tune->waves_per_block)))
-    return false;
-  const int64_t block = bits == 4 ? 32 : 16;  // the general kernels' row blocks
-  const int64_t size = (M + block - 1) / block * block * N * K;
-  return K > 4096 || size > (bits == 4 ? 1ll << 29 : 1ll << 28);
+  return gemm_shape(M, K, N, gs) &&
+         (!tune || (tune->path == 0 && !tune->tiles_per_wave && !tune->waves_per_block)) &&
+         !small_product(M, K, N, bits);
 }
 
 extern "C" size_t dfmi_qmm_workspace_bytes_ex(int64_t M, int64_t K, int64_t N, int group_size,
@@ -1088,7 +1097,7 @@ extern "C" int dfmi_qmm_gemm_plan(int64_t M, int64_t K, const int64_t* Ns, int n
   }
   *tile_rows = *tile_cols = *k_splits = 0;
   if (nseg == 1 ? Ns[0] > 0 && use_gemm(M, K, Ns[0], group_size, bits, nullptr)
-                : use_gemm_multi(M, K, Ns, nseg, group_size))
+                : use_gemm_multi(M, K, Ns, nseg, group_size, bits))
     gemm_plan_query(M, K, Ns, nseg, tile_rows, tile_cols, k_splits);
   return DFMI_OK;
 }
@@ -1327,7 +1336,7 @@ extern "C" size_t dfmi_qmm_multi_workspace_bytes(int64_t M, int64_t K, const int
   size_t ws = 0;
   for (int i = 0; i < nseg; ++i)
     ws = std::max(ws, dfmi_qmm_workspace_bytes_ex(M, K, Ns[i], group_size, bits, nullptr));
-  if (use_gemm_multi(M, K, Ns, nseg, group_size))
+  if (use_gemm_multi(M, K, Ns, nseg, group_size, bits))
     ws = std::max(ws, gemm_multi_workspace_bytes(M, K, Ns, nseg, group_size));
   return ws;
 }
@@ -1389,7 +1398,7 @@ static int qmm_multi(const void* x, int x_dtype, const dfmi_qmm_segment* segs, i
     return launch_streaming(x, x_dtype, m, M, K, cols, group_size, bits, nullptr, workspace,
                             workspace_bytes, static_cast<hipStream_t>(stream));
   }
-  if (use_gemm_multi(M, K, Ns, nseg, group_size)) {
+  if (use_gemm_multi(M, K, Ns, nseg, group_size, bits)) {
     const int rc = gemm_launch(x, x_dtype, segs, nseg, fused, 0, M, K, group_size, bits,
                                workspace, workspace_bytes, static_cast<hipStream_t>(stream));
     if (rc != kGemmNotTaken) return rc;

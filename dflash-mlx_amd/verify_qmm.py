@@ -215,7 +215,7 @@ class LaunchRecord:
     matrices, their tables side by side.  The record keeps these tensors and
     the stream's workspace alive while it exists; run it only on the stream
     it was prepared for (the workspace is that stream's).  Beyond 32 rows a
-    run is one :func:`qmm_multi_launch`, with scratch of its own."""
+    run that needs scratch takes it for itself, and no table of the record."""
 
     __slots__ = ("_buf", "ptr", "_keep", "M", "Ns", "dtype", "_many")
 
@@ -247,7 +247,7 @@ class LaunchRecord:
             ns = (ctypes.c_int64 * n)(*Ns)
             need = int(lib.dfmi_qmm_multi_workspace_bytes(M, K, ns, n, int(group_size),
                                                           int(bits)))
-        many = _runtime.many_rows(M)  # (each run brings scratch of its own)
+        many = need > 0 and _runtime.many_rows(M)  # (each run brings its scratch)
         ws, ws_bytes = _runtime.workspace(dev, need) if need and not many else (0, 0)
         buf = ctypes.create_string_buffer(_lib.DFMI_QMM_RECORD_BYTES + 16)
         ptr = (ctypes.addressof(buf) + 15) // 16 * 16
@@ -259,24 +259,39 @@ class LaunchRecord:
         keep.append(fused)
         self._buf, self.ptr, self._keep = buf, ptr, keep
         self.M, self.Ns, self.dtype = M, Ns, dtype
-        self._many = (([(m[0], m[1], m[2]) for m in mats], int(group_size), int(bits))
-                      if many else None)
+        self._many = None
+        if many:
+            for s in segs:
+                s.sb_pairs = None
+            self._many = (segs, n, int(M), int(K), int(group_size), int(bits), need)
 
     def run(self, x2: torch.Tensor, ys, stream: int) -> None:
         """Launch on ``x2 [M, K]`` (contiguous, 16-byte aligned) into ``ys``."""
         if self._many is not None:
             dev = x2.device
             if int(stream) == current_stream(dev.index):
-                qmm_multi_launch(x2, *self._many, outs=ys)
+                self._run_many(x2, ys)
             else:
                 with torch.cuda.stream(torch.cuda.ExternalStream(int(stream), device=dev) if stream
                                        else torch.cuda.default_stream(dev)):
-                    qmm_multi_launch(x2, *self._many, outs=ys)
+                    self._run_many(x2, ys)
             return
         p = [y.data_ptr() for y in ys] + [None] * (4 - len(ys))
         status = _lib.load().dfmi_qmm_run(self.ptr, x2.data_ptr(), p[0], p[1], p[2], p[3], stream)
         if status:
             _lib.check(status, "dfmi_qmm_run")
+
+    def _run_many(self, x2: torch.Tensor, ys) -> None:
+        segs, n, M, K, group_size, bits, need = self._many
+        segs = type(segs).from_buffer_copy(segs)  # (several threads may run a record)
+        for s, y in zip(segs, ys):
+            s.y = y.data_ptr()
+        scratch = _runtime.call_scratch(x2.device, need)
+        status = _lib.load().dfmi_qmm_affine_multi(
+            x2.data_ptr(), _runtime.dtype_code(self.dtype), segs, n, M, K, group_size, bits,
+            scratch.data_ptr(), need, _runtime.stream_ptr(x2.device))
+        if status:
+            _lib.check(status, "dfmi_qmm_affine_multi")
 
 
 def _prepare(x, w, scales, biases):

@@ -248,8 +248,9 @@ size_t dfmi_qmm_noalloc_scratch_bytes(void);
  * an MLP (dflash_mlx/verify_linear.py:266-286, one call per
  * VerifyQuantizedLinear) -- so that the layer pays one launch, one pipeline
  * fill and one grid for them: the row blocks of all W_i form one streaming
- * grid.  At M > 32 two or three matrices (each N a multiple of 4) form one
- * matrix-core grid likewise, given the workspace or their pair tables.  Other
+ * grid.  At M > 32 two or three matrices (each N a multiple of 4; not two
+ * small products with K up to 768) form one matrix-core grid likewise, given
+ * the workspace or their pair tables.  Other
  * shapes (K % 256 != 0, ...) run as nseg dfmi_qmm_affine calls on the stream,
  * in order.  Each y_i is within fp32 summation order of what dfmi_qmm_affine
  * returns for W_i alone (the two may split K differently); the result does not

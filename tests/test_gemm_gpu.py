@@ -220,7 +220,7 @@ def test_rows_with_infinities_stay_apart(dev):
 
 
 @pytest.mark.parametrize("M,K,Ns,gs,bits,dtype", [
-    (33, 64, (4, 260), 32, 4, "bf16"), (77, 1152, (132, 4, 388), 64, 4, "f16"),
+    (33, 64, (4, 260, 4), 32, 4, "bf16"), (77, 800, (4, 260), 32, 4, "bf16"), (77, 1152, (132, 4, 388), 64, 4, "f16"),
     (200, 640, (512, 128), 128, 8, "bf16"), (65, 4096, (256, 260, 64), 64, 4, "bf16"),
 ])
 def test_matrices_in_one_launch(dev, M, K, Ns, gs, bits, dtype):
