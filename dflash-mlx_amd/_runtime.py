@@ -6,6 +6,7 @@ arithmetic on the verify path happens in libdfmi.so.
 
 from __future__ import annotations
 
+import copy
 import threading
 import weakref
 from typing import Optional, Tuple
@@ -223,6 +224,9 @@ class _Built:
             torch.cuda.current_stream(self.device).wait_event(self.event)
             self.streams.add(st)
         return self.table
+
+    def __deepcopy__(self, memo) -> "_Built":  # (of a module: events are not copied)
+        return _Built(copy.deepcopy(self.get(), memo))
 
 
 class _PairCache:

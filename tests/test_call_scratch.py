@@ -8,6 +8,7 @@ stream."""
 
 from __future__ import annotations
 
+import copy
 import threading
 
 import pytest
@@ -172,6 +173,8 @@ def test_tables_are_waited_for_once_per_stream(monkeypatch):
         at.update(stream=stream, capturing=capturing)
         assert built.get() is table
     assert waits == [2, 3]
+    twin = copy.deepcopy(built)  # (as with the module that holds it)
+    assert twin.table is not table and torch.equal(twin.get(), table)
 
 
 def test_expert_tensors_on_another_device(library):

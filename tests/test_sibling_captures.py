@@ -5,6 +5,8 @@ launch on another stream than the install's waits for the tables."""
 
 from __future__ import annotations
 
+import copy
+
 import pytest
 import torch
 
@@ -73,6 +75,26 @@ def test_each_launch_prepared_waits_for_its_table(monkeypatch):
     for st in (5, 5, 6):
         grp._record(16, st, x, (0, 1))
     assert gets == ["a", "b"] * 2
+
+
+@pytest.mark.gpu
+def test_deepcopy_of_an_installed_model(dev):
+    """A model is copied with its tables, also after calls of every kind."""
+    from torch import nn
+
+    root = nn.Module()
+    root.mlp = nn.Module()
+    for name in ("gate_proj", "up_proj"):
+        setattr(root.mlp, name, vl.QuantizedLinear.from_linear(
+            nn.Linear(1024, 256, bias=False, device=dev), 64, 4, torch.bfloat16))
+    vl.install_verify_linears(root, enable_qmm=True)
+    x = torch.randn((16, 1024), device=dev).to(torch.bfloat16)
+    want = root.mlp.gate_proj(x), root.mlp.up_proj(x)
+    twin = copy.deepcopy(root)
+    got = twin.mlp.gate_proj(x), twin.mlp.up_proj(x)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    state = twin.mlp.gate_proj._verify_state
+    assert torch.equal(state.built.get()[:, :256], state.pairs)
 
 
 @pytest.mark.gpu
