@@ -66,9 +66,9 @@ def _pairs_table(pairs: Optional[torch.Tensor], scales: torch.Tensor, biases: to
     shape takes one, it is the cached table of these scales / biases (few
     pairs: built on first use, never during graph capture) or, for many pairs,
     one built for the call from the scales as they are, where that pays."""
-    E, _, G = (int(d) for d in scales.shape)
-    cols = 2 * N if up is not None else N
     if pairs is not None:
+        E, _, G = (int(d) for d in scales.shape)
+        cols = 2 * N if up is not None else N
         _runtime.require_device(pairs, "pairs")
         if (pairs.dtype != torch.int32 or tuple(pairs.shape) != (E, G, cols)
                 or not pairs.is_contiguous()):
@@ -78,7 +78,7 @@ def _pairs_table(pairs: Optional[torch.Tensor], scales: torch.Tensor, biases: to
         return None
     if few:
         return _runtime.PAIRS.get(scales, biases, up, experts=True)
-    if not _table_pays(P, K, N, E, group_size, up is not None):
+    if not _table_pays(P, K, N, int(scales.shape[0]), group_size, up is not None):
         return None
     return _runtime.build_moe_pairs(scales, biases, *(up if up is not None else ()))
 
